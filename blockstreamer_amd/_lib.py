@@ -93,8 +93,18 @@ _SIGNATURES = {
         _int, _i64, _f32,                          # causal, window, scaling
         _ptr, _ptr, _ptr, _ptr, _ptr,              # grad_q, grad_k, grad_v, row_dot, stream
     ],
+    "bsa_attention_bwd_workspace_bytes": [_i64, _i64, _i64, _i64, _i64, _int, _i64],
+    "bsa_attention_bwd_split": [
+        _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,  # grad_out, q, k, v (each with strides)
+        _ptr, _ptr, _ptr,                          # out, out strides, lse
+        _i64, _i64, _i64, _i64, _i64, _i64,        # B, Tq, Tk, Hq, Hkv, head_dim
+        _int, _i64, _f32,                          # causal, window, scaling
+        _ptr, _ptr, _ptr, _ptr,                    # grad_q, grad_k, grad_v, row_dot
+        _ptr, _i64, _ptr,                          # workspace, bytes, stream
+    ],
 }
-_RESTYPE = {"bsa_last_error": ctypes.c_char_p, "bsa_attention_split_workspace_bytes": ctypes.c_int64}
+_RESTYPE = {"bsa_last_error": ctypes.c_char_p, "bsa_attention_split_workspace_bytes": ctypes.c_int64,
+            "bsa_attention_bwd_workspace_bytes": ctypes.c_int64}
 
 _lib = None
 

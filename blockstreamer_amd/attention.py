@@ -52,6 +52,12 @@ def _split_bytes(B: int, Tq: int, Tk: int, Hq: int, Hkv: int, causal: int, windo
     return int(_lib.lib().bsa_attention_split_workspace_bytes(B, Tq, Tk, Hq, Hkv, causal, window))
 
 
+@functools.lru_cache(maxsize=256)
+def _bwd_split_bytes(B: int, Tq: int, Tk: int, Hq: int, Hkv: int, causal: int, window: int) -> int:
+    """Workspace of the row-split backward for a shape (0: not split), a function of the shape."""
+    return int(_lib.lib().bsa_attention_bwd_workspace_bytes(B, Tq, Tk, Hq, Hkv, causal, window))
+
+
 def attention_forward(query: Tensor, key: Tensor, value: Tensor, sinks: Tensor | None, scaling: float,
                       causal: bool = False, window: int = 0, return_lse: bool = False):
     """``softmax([q k^T * scaling | sink]) v`` per head, the sink column dropped.
@@ -117,13 +123,18 @@ def attention_backward(grad_out: Tensor, query: Tensor, key: Tensor, value: Tens
     dv = torch.empty_like(dk)
     # per row R = t * (Hq / Hkv) + i of key head hk: (L, D), D = grad_out . out
     row_stats = torch.empty(B, Hkv, Tq * (Hq // Hkv), 2, dtype=torch.float32, device=dev)
+    # short sequences split the rows that see each key block over several
+    # workgroups; the library says from the shape how much workspace that takes
+    ws_bytes = _bwd_split_bytes(B, Tq, Tk, Hq, Hkv, 1 if causal else 0, int(window))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
     with torch.cuda.device(dev):
-        _lib.call("bsa_attention_bwd",
+        _lib.call("bsa_attention_bwd_split",
                   g.data_ptr(), _strides(g, 1, 2), q.data_ptr(), _strides(q, 2, 1),
                   k.data_ptr(), _strides(k, 2, 1), v.data_ptr(), _strides(v, 2, 1),
                   o.data_ptr(), _strides(o, 1, 2), lse.data_ptr(),
                   B, Tq, Tk, Hq, Hkv, D, 1 if causal else 0, int(window), float(scaling),
-                  dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), row_stats.data_ptr(), _lib.stream_handle(dev))
+                  dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), row_stats.data_ptr(),
+                  ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_handle(dev))
     dsinks = None
     if sinks_grad:
         # d sink[h] = -sum_t p_sink[t] D[t], p_sink = 2^(sink log2(e) - lse)

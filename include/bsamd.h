@@ -502,6 +502,36 @@ int bsa_attention_bwd(const void *grad_out, const int64_t *grad_strides,
                       float scaling, void *grad_q, void *grad_k, void *grad_v,
                       float *row_stats, void *stream);
 
+/*
+ * Workspace bytes of bsa_attention_bwd_split for a shape (0: that shape is not
+ * split): when a key block has enough rows, the rows that see it are split
+ * over up to 32 workgroups.  A function of the shape only.  Replaces no
+ * reference interface.
+ */
+int64_t bsa_attention_bwd_workspace_bytes(int64_t B, int64_t Tq, int64_t Tk,
+                                          int64_t Hq, int64_t Hkv, int causal,
+                                          int64_t window);
+
+/*
+ * bsa_attention_bwd (the same arguments and meaning,
+ * modeling_gpt_oss.py:235-264) with the rows of each key block split: the
+ * shares' float32 sums of grad_k and grad_v go to the workspace (>= the query
+ * above, 16-byte aligned; may be NULL when that is 0) and a further launch
+ * adds them in a fixed order (deterministic; equal to bsa_attention_bwd to
+ * float rounding).
+ */
+int bsa_attention_bwd_split(const void *grad_out, const int64_t *grad_strides,
+                            const void *q, const int64_t *q_strides,
+                            const void *k, const int64_t *k_strides,
+                            const void *v, const int64_t *v_strides,
+                            const void *out, const int64_t *out_strides,
+                            const float *lse, int64_t B, int64_t Tq,
+                            int64_t Tk, int64_t Hq, int64_t Hkv,
+                            int64_t head_dim, int causal, int64_t window,
+                            float scaling, void *grad_q, void *grad_k,
+                            void *grad_v, float *row_stats, void *workspace,
+                            int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

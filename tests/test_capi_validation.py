@@ -259,3 +259,24 @@ def test_attention_split_workspace_follows_the_shape():
     assert f(1, 1, 448, 64, 8, 1, 0) == 0             # 7 key tiles: too few
     assert f(1, 1, 449, 64, 8, 1, 0) == 4 * 64 * 64 * 4 + 4 * 64 * 2 * 4  # 8 tiles: 4 shares
     assert f(2, 4, 1000, 64, 8, 1, 0) > 0
+
+
+def test_attention_bwd_split_workspace_follows_the_shape():
+    """Shares x (dk, dv) x key heads x keys x 64 floats; none where the key blocks fill the chip or rows are few."""
+    f = _lib.lib().bsa_attention_bwd_workspace_bytes
+    part = lambda n, B, Hkv, Tk: n * 2 * B * Hkv * Tk * 64 * 4  # noqa: E731
+    assert f(1, 8192, 8192, 64, 8, 1, 0) == part(4, 1, 8, 8192)
+    assert f(1, 4096, 4096, 64, 8, 1, 0) == part(8, 1, 8, 4096)
+    assert f(1, 2048, 2048, 64, 8, 1, 0) == part(8, 1, 8, 2048)
+    assert f(1, 8192, 8192, 64, 8, 1, 128) == 0
+    assert f(1, 32768, 32768, 64, 8, 1, 0) == 0       # 2048 key blocks
+    assert f(1, 64, 64, 64, 8, 1, 0) == 0             # 16 units of rows: one share
+    assert f(0, 64, 64, 64, 8, 1, 0) == 0
+
+
+@pytest.mark.parametrize("ws,nbytes", [(None, 1 << 40), (FAKE, 4096), (FAKE + 8, 1 << 40)])
+def test_attention_bwd_split_refuses_a_bad_workspace(ws, nbytes):
+    a = _attn_bwd_args(Tq=2048, Tk=2048)
+    args = a[:-1] + (ws, nbytes, None)
+    assert _lib.lib().bsa_attention_bwd_split(*args) == _lib.BSA_EINVAL
+    assert b"workspace" in _lib.lib().bsa_last_error()

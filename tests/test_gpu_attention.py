@@ -326,3 +326,79 @@ def test_forward_backward_2048_vs_float32(device, window):
     out2.backward(dout)
     torch.cuda.synchronize()
     assert torch.equal(out, out2) and torch.equal(qg.grad, q2.grad) and torch.equal(kg.grad, k2.grad)
+
+
+# row splits of dk/dv, key blocks and units that end early, groups that do and
+# do not divide a 32-row unit, offset queries, windows shorter and longer than a block
+BWD_SPLIT_CASES = [
+    # B, Hq, Hkv, Tq, Tk, causal, window, row splits expected
+    (1, 8, 1, 512, 512, True, 0, True),
+    (1, 6, 2, 601, 601, True, 0, True),     # G = 3
+    (2, 8, 8, 1101, 1101, True, 0, True),   # G = 1
+    (1, 32, 2, 130, 257, True, 0, True),    # G = 16
+    (1, 64, 1, 40, 129, False, 0, True),    # G = 64
+    (1, 10, 2, 257, 300, False, 0, True),   # G = 5
+    (1, 16, 2, 300, 300, True, 31, True),
+    (1, 16, 2, 300, 500, True, 200, True),
+    (1, 64, 8, 31, 31, True, 0, False),
+    (1, 64, 8, 33, 127, True, 64, False),
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Tq,Tk,causal,window,split", BWD_SPLIT_CASES)
+def test_backward_row_splits_vs_single_share_and_oracle(device, B, Hq, Hkv, Tq, Tk, causal, window, split):
+    announce(f"attention bwd splits B={B} Hq={Hq} Hkv={Hkv} Tq={Tq} Tk={Tk} causal={causal} window={window}")
+    lib = A._lib.lib()
+    nbytes = lib.bsa_attention_bwd_workspace_bytes(B, Tq, Tk, Hq, Hkv, int(causal), window)
+    assert (nbytes > 0) == split
+    q, k, v, s = _inputs(B, Hq, Hkv, Tq, Tk, device, seed=Tq + Hq, layout="bhtd" if Tq % 2 else "bthd")
+    dout = torch.randn(B, Tq, Hq, 64, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16).to(device)
+    out, lse = A.attention_forward(q, k, v, s, 0.125, causal, window, return_lse=True)
+    got = A.attention_backward(dout, q, k, v, s, out, lse, 0.125, causal, window)
+    # the same gradients with one share per key block
+    dq = torch.empty(B, Tq, Hq, 64, dtype=torch.bfloat16, device=device)
+    dk = torch.empty(B, Tk, Hkv, 64, dtype=torch.bfloat16, device=device)
+    dv = torch.empty_like(dk)
+    stats = torch.empty(B, Hkv, Tq * (Hq // Hkv), 2, dtype=torch.float32, device=device)
+    A._lib.call("bsa_attention_bwd", dout.data_ptr(), A._strides(dout, 1, 2), q.data_ptr(), A._strides(q, 2, 1),
+                k.data_ptr(), A._strides(k, 2, 1), v.data_ptr(), A._strides(v, 2, 1), out.data_ptr(),
+                A._strides(out, 1, 2), lse.data_ptr(), B, Tq, Tk, Hq, Hkv, 64, int(causal), window, 0.125,
+                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), stats.data_ptr(), A._lib.stream_handle(dq.device))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0].transpose(1, 2), dq)
+    for name, a, b in (("dk", got[1], dk.transpose(1, 2)), ("dv", got[2], dv.transpose(1, 2))):
+        # the same float32 terms in another order, then one bf16 rounding: at
+        # most a flipped rounding here and there (half an ulp is 2^-9)
+        assert _rel_l2(a, b) <= 2.0 ** -9, name
+        if not split:
+            assert torch.equal(a, b), name
+    qr, kr, vr = (t.detach().cpu().double().requires_grad_(True) for t in (q, k, v))
+    ref = oracle.attention_ref(qr, kr, vr, s.cpu().double(), 0.125, causal=causal, window=window)
+    ref.backward(dout.double().cpu())
+    for name, a, want in zip(("dq", "dk", "dv"), got, (qr.grad, kr.grad, vr.grad)):
+        assert _rel_l2(a, want) <= BWD_REL_L2, name
+
+
+def test_attention_far_strides(device):
+    """Row strides past the 32-bit offset of the DMA's near form (2^24 bytes): the same bits as contiguous."""
+    announce("attention far strides")
+    B, Hq, Hkv, T = 1, 8, 1, 70
+    q, k, v, s = _inputs(B, Hq, Hkv, T, T, device, seed=8)
+    dout = torch.randn(B, T, Hq, 64, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(device)
+    row = (1 << 23) + 64  # elements
+
+    def far(t, heads):  # [B, heads, T, 64] view with T rows `row` elements apart
+        buf = torch.zeros(T * row, dtype=torch.bfloat16, device=device)
+        view = buf.as_strided((B, heads, T, 64), (T * row, 64, row, 1))
+        view.copy_(t)
+        return view
+
+    want_out, lse = A.attention_forward(q, k, v, s, 0.125, True, 0, return_lse=True)
+    want = A.attention_backward(dout, q, k, v, s, want_out, lse, 0.125, True, 0)
+    fq, fk, fv = far(q, Hq), far(k, Hkv), far(v, Hkv)
+    out, lse2 = A.attention_forward(fq, fk, fv, s, 0.125, True, 0, return_lse=True)
+    got = A.attention_backward(dout, fq, fk, fv, s, out, lse2, 0.125, True, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want_out)
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a, b)
