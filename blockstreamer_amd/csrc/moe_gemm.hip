@@ -808,13 +808,17 @@ __global__ __launch_bounds__(256, 3) void moe_stream_parts_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Persistent weight-streaming kernel (decode) for a K = 32*G known at compile
-// time.  Persistent workgroups (WPC per CU) each walk a contiguous run of
-// work items; an item is 16 weight rows (one 16x16x32 MFMA column block) of
-// one expert against one 16-row pass of that expert's sorted rows, items
+// Persistent weight-streaming kernel (decode and short prompts) for a K =
+// 32*G known at compile time.  Persistent workgroups, two per CU, each walk a
+// contiguous run of work items; an item is 16 weight rows (one 16-column MFMA
+// block) of one expert against one pass of that expert's sorted rows, items
 // ordered by (hit expert, pass, weight-row slice).  Consecutive items of a
 // workgroup share the expert, so the A operands stay in registers and are
 // reloaded only when the (expert, pass) changes.
+//
+// A pass is 16 rows per row group, RG groups of four waves per workgroup: every
+// item's weights are read once for all of a pass's rows, so RG is the number
+// of 16-row blocks that share one read of the weights (ps_row_groups).
 //
 // The items' packed bytes stream through a ring of NB LDS slots by
 // global_load_lds DMA, NB - 1 items ahead of the computation.  A slot holds
@@ -823,20 +827,23 @@ __global__ __launch_bounds__(256, 3) void moe_stream_parts_kernel(GemmArgs a) {
 // different bank groups.  The last part has 16 - G % 16 unused slots per row
 // (groups past G); they carry the item's 16*G scale bytes and its 16 bias
 // values, chunk j (16 bytes) in row j / UN, slot (G % 16 + j % UN) ^ (j / UN).
-// So every wave issues exactly G/16 DMA instructions per item and "item i
-// has landed" is vmcnt <= (G/16) * (items issued after i).  The epilogue's
+// So every wave issues exactly NP / RG DMA instructions per item (row group r
+// the parts p = r mod RG) and "item i has landed" is vmcnt <= (NP / RG) * (items
+// issued after i).  The epilogue's
 // stores also count in vmcnt; leaving them out of that bound only makes the
 // wait stricter.  A reload of the A operands waits for everything.
 //
-// Waves split K as the part kernel does (wave w takes groups 16p + 4w + c).
-// All four partial sums go through LDS; wave w finishes rows 4c + w, adding
-// the partials in wave order, so results equal the part kernel's bit for bit.
+// A row group's waves split K as the part kernel does (wave w takes groups 16p +
+// 4w + c).  The four partial sums go through LDS; wave w finishes rows 4c + w,
+// adding the partials in wave order, so a row's result depends neither on its
+// pass nor on RG.
 // LDS reads of the ring are inline assembly: the compiler cannot tell which
 // slot a computed address falls in, and for an ordinary LDS load it would
 // wait for every global_load_lds in flight (vmcnt(0)), draining the ring.
 // ---------------------------------------------------------------------------
-constexpr int PS_TEAM_NB = 3;   // ring slots per team
-constexpr int PS_TEAMS = 1;     // teams per workgroup (1: two workgroups per CU)
+// Ring slots per row group: 147 KiB of weights in flight per CU, in two rings of
+// three slots (RG = 1, two workgroups per CU) or one of six (RG = 2).
+constexpr int PS_NB = 3;
 
 template <int G>
 struct PsCfg {
@@ -856,7 +863,7 @@ __host__ __device__ constexpr uint32_t ps_chunk_off(int j, int b) {
 }
 
 // Position in a workgroup's item sequence: hit-list entry h (expert e with
-// cnt rows), pass (16-row block of those rows), slice s (16 weight rows).
+// cnt rows), pass (ROWS of those rows), slice s (16 weight rows).
 struct PsIt {
   int h, pass, s, e, cnt;
 };
@@ -867,20 +874,22 @@ __device__ __forceinline__ void ps_entry(PsIt& it, const int* sHit) {
   it.cnt = v >> 10;
 }
 
+template <int ROWS>
 __device__ __forceinline__ void ps_next(PsIt& it, const int* sHit, int S, int nhit) {
   if (++it.s == S) {
     it.s = 0;
-    if (++it.pass * 16 >= it.cnt) {
+    if (++it.pass * ROWS >= it.cnt) {
       it.pass = 0;
       if (++it.h < nhit) ps_entry(it, sHit);
     }
   }
 }
 
-// DMA of one item (expert e, weight rows n0 .. n0+15) into slot sb: G/16
-// instructions per wave, wave w filling rows 4w .. 4w+3 of every part.
-template <int G>
-__device__ __forceinline__ void ps_issue(const GemmArgs& a, uint8_t* sb, int e, int n0, int wave,
+// DMA of one item (expert e, weight rows n0 .. n0+15) into slot sb: NP / RG
+// instructions per wave, wave w of row group rg filling rows 4w .. 4w+3 of the
+// parts p = rg mod RG.
+template <int G, int RG>
+__device__ __forceinline__ void ps_issue(const GemmArgs& a, uint8_t* sb, int e, int n0, int rg, int wave,
                                          int lane, int eb) {
   using C = PsCfg<G>;
   const int64_t r0 = (int64_t)e * a.N + n0;
@@ -888,8 +897,10 @@ __device__ __forceinline__ void ps_issue(const GemmArgs& a, uint8_t* sb, int e, 
   const uint8_t* gS = a.Bs + r0 * G;
   const int row = 4 * wave + (lane >> 4);
   const int sl = (lane & 15) ^ row;
+  static_assert(C::NP % RG == 0, "the parts split evenly over the row groups");
 #pragma unroll
-  for (int p = 0; p < C::NP; ++p) {
+  for (int i = 0; i < C::NP / RG; ++i) {
+    const int p = i * RG + rg;
     const uint8_t* src = gB + bq_off(a.kp, row, 16 * p + sl, G);
     if (p == C::NP - 1 && 16 * p + sl >= G) {
       // a spare slot: scale chunk j, then the bias chunks, else anything valid
@@ -987,18 +998,18 @@ __device__ __forceinline__ f32x4_t mfma_mx16(const i32x8_t& a, const i32x8_t& b,
   }
 }
 
-// FP8 A operands (hi and lo) of this lane for pass `pass` of an expert whose
-// sorted rows start at row0, for the 16x16x128 block-scaled MFMA over the
+// FP8 A operands (hi and lo) of this lane for the 16 rows from row pass0 of an
+// expert whose sorted rows start at row0, for the 16x16x128 block-scaled MFMA over the
 // 4-group window 16p + 4*wave of part p: lane group c holds k 16c .. 16c+15
 // (bytes 0-15) and 64+16c .. 64+16c+15 (bytes 16-31) of the window and
 // supplies the scale of window block c.  Rows past cnt repeat the last valid
 // row (their outputs are never stored).  Scale bytes of parts 0-3 / 4-5 are
 // packed into sh[0] / sh[1] (byte p % 4), likewise sl.
 template <int G>
-__device__ __forceinline__ void ps_load_a_raw(const GemmArgs& a, int row0, int cnt, int pass, int col, int c,
+__device__ __forceinline__ void ps_load_a_raw(const GemmArgs& a, int row0, int cnt, int pass0, int col, int c,
                                               int wave, u32x4_t (&raw)[PsCfg<G>::NP][4]) {
   constexpr int NP = PsCfg<G>::NP;
-  const int r = min(pass * 16 + col, cnt - 1);
+  const int r = min(pass0 + col, cnt - 1);
   const int64_t pos = row0 + r;
   const int64_t src = a.row_pair ? (int64_t)(a.row_pair[pos] / a.topk) : pos;
   const uint16_t* arow = a.A + src * a.lda;
@@ -1092,25 +1103,20 @@ __device__ __forceinline__ void ps_epilogue(const GemmArgs& a, const f32x4_t* sR
   }
 }
 
-// TEAMS teams of four waves per workgroup, each team with its own
-// PS_TEAM_NB-slot ring and its own share of the workgroup's contiguous run of
-// items.  TEAMS = 2: one 512-thread workgroup per CU whose teams meet at every
-// barrier, so both halves of a CU finish together.  TEAMS = 1: two
-// independent 256-thread workgroups per CU (more overlap between them, but
-// the CU serves them unevenly).
-template <int EPI, int G, int TEAMS>
-__global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_kernel(GemmArgs a) {
+template <int EPI, int G, int RG>
+__global__ __launch_bounds__(256 * RG, 2) void moe_stream_persist_kernel(GemmArgs a) {
   using C = PsCfg<G>;
   constexpr int NP = C::NP;
-  constexpr int NB = PS_TEAM_NB;
-  constexpr int NT = 256 * TEAMS;                            // threads
+  constexpr int NB = PS_NB * RG;
+  constexpr int DPI = NP / RG;                               // DMA instructions per wave and item
+  constexpr int ROWS = 16 * RG;                              // rows per pass
+  constexpr int NT = 256 * RG;                               // threads
   constexpr int MAXE = NT;                                   // experts the hit-list tables hold
   static_assert(NP == 6, "the ring reads below are written out for six parts");
-  extern __shared__ __align__(1024) uint8_t ring[];          // TEAMS x NB slots
-  __shared__ f32x4_t sRed[TEAMS * 4 * 64];                   // partial sums, [team][wave][lane]
+  extern __shared__ __align__(1024) uint8_t ring[];          // NB slots
+  __shared__ f32x4_t sRed[RG * 4 * 64];                      // partial sums, [row group][wave][lane]
   __shared__ int sHit[MAXE];                                 // e | cnt << 10, in expert order
   __shared__ int sRow0[MAXE];                                // first sorted row of entry h
-  __shared__ int sSeg[2];                                    // each team's steps to its next reload
   int* sScan = reinterpret_cast<int*>(sRed);                 // prologue scratch: NT + 2 ints
   int* sHPre = sScan + NT + 2;                               // prologue: passes before entry h
 
@@ -1127,8 +1133,8 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
     __syncthreads();  // this workgroup's writes are visible to its reads below
   }
   const int lane = tid & 63;
-  const int team = TEAMS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
-  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);   // wave within the team
+  const int rg = RG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;   // row group
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);        // wave within it
   const int col = lane & 15;
   const int c = lane >> 4;
   const int S = a.N / 16;
@@ -1137,7 +1143,7 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
   // --- hit list: experts with rows, their pass prefix, in expert order -----
   const int cnt_t = tid < a.E ? a.counts[tid] : 0;
   const int off_t = tid < a.E ? a.offsets[tid] : 0;
-  const int mine = (cnt_t > 0 ? 1 : 0) | (((cnt_t + 15) >> 4) << 16);
+  const int mine = (cnt_t > 0 ? 1 : 0) | (((cnt_t + ROWS - 1) / ROWS) << 16);
   // inclusive scan: shuffles within each wave, then the wave totals
   int incl = mine;
 #pragma unroll
@@ -1167,50 +1173,39 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
   const int n_items = min(total - start, chunk);
   __syncthreads();
   if (n_items <= 0) return;
-  // the workgroup's run: team 0 takes the first half, team 1 the rest
-  const int half = TEAMS == 2 ? (n_items + 1) >> 1 : n_items;
-  const int tstart = start + (team ? half : 0);
-  const int tn = team ? n_items - half : half;   // team 1 may have one item less (or none)
-  // entries holding each team's first pass
-  if (tid < 2) sScan[NT + tid] = 0;
-  __syncthreads();
+  // the entry holding the first pass of the workgroup's run
+  const int tq0 = start / S;
   if (tid < nhit) {
-    const int np = ((sHit[tid] >> 10) + 15) >> 4;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int q = min(start + (t ? half : 0), total - 1) / S;
-      if (sHPre[tid] <= q && q < sHPre[tid] + np) sScan[NT + t] = tid;
-    }
+    const int np = ((sHit[tid] >> 10) + ROWS - 1) / ROWS;
+    if (sHPre[tid] <= tq0 && tq0 < sHPre[tid] + np) sScan[NT] = tid;
   }
   __syncthreads();
   PsIt ci;
-  const int tq0 = min(tstart, total - 1) / S;
-  ci.h = __builtin_amdgcn_readfirstlane(sScan[NT + team]);
+  ci.h = __builtin_amdgcn_readfirstlane(sScan[NT]);
   ps_entry(ci, sHit);
   ci.pass = tq0 - __builtin_amdgcn_readfirstlane(sHPre[ci.h]);
-  ci.s = min(tstart, total - 1) - tq0 * S;
+  ci.s = start - tq0 * S;
   PsIt ii = ci;
   __syncthreads();  // the prologue scratch becomes the partial-sum buffer
 
-  uint8_t* tring = ring + team * (NB * C::SLOT);
-  f32x4_t* tred = sRed + team * 256;
+  f32x4_t* tred = sRed + rg * 256;
 
-  // --- A operands of the first group (loaded before any DMA is in flight),
-  // then the team's first NB items' DMA, then the quantisation -------------
+  // --- A operands of the first pass (loaded before any DMA is in flight),
+  // then the first NB items' DMA, then the quantisation ---------------------
   i32x8_t ah[NP], al[NP];   // FP8 hi / lo activation operands
   uint32_t sah[2], sal[2];   // their scale bytes, byte p % 4 of word p / 4
-  int row0 = 0;
-  if (tn > 0) {
-    row0 = __builtin_amdgcn_readfirstlane(sRow0[ci.h]);
+  int row0 = __builtin_amdgcn_readfirstlane(sRow0[ci.h]);
+  bool live = ci.pass * ROWS + 16 * rg < ci.cnt;  // this row group has rows in the pass
+  {
     u32x4_t raw[NP][4];
-    ps_load_a_raw<G>(a, row0, ci.cnt, ci.pass, col, c, wave, raw);
+    if (live) ps_load_a_raw<G>(a, row0, ci.cnt, ci.pass * ROWS + 16 * rg, col, c, wave, raw);
     wait_vmcnt<0>();
-    const int npre = min(NB, tn);
+    const int npre = min(NB, n_items);
     for (int j = 0; j < npre; ++j) {
-      ps_issue<G>(a, tring + j * C::SLOT, ii.e, ii.s * 16, wave, lane, eb);
-      ps_next(ii, sHit, S, nhit);
+      ps_issue<G, RG>(a, ring + j * C::SLOT, ii.e, ii.s * 16, rg, wave, lane, eb);
+      ps_next<ROWS>(ii, sHit, S, nhit);
     }
-    ps_quant_a<G>(raw, c, wave, ah, al, sah, sal);
+    if (live) ps_quant_a<G>(raw, c, wave, ah, al, sah, sal);
   }
   const uint32_t boff = (uint32_t)(col * 256 + (((4 * wave + c) ^ col) * 16));
   uint32_t soff[NP];  // this lane's scale byte of group 16p + 4*wave + c, row col
@@ -1220,38 +1215,25 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
     soff[p] = ps_chunk_off<G>(o >> 4, o & 15);
   }
   const uint32_t bofs = ps_chunk_off<G>(G + (col * eb) / 16, ((col * eb) & 15) & ~3);
-  const uint32_t ring0 = lds_addr(tring);
+  const uint32_t ring0 = lds_addr(ring);
 
-  // Per step k (one item per team, team item k): wait for its DMA, barrier,
-  // finish the epilogue of item k-1 (its partial sums were written before
-  // this barrier), read item k's slot into registers, barrier (the slot is
-  // free), refill the slot with item k+NB, and only then multiply.  Segments
-  // end where either team's (expert, pass) changes; that team then reloads
-  // its A operands (waiting for everything it has in flight).
-  const int nsteps = half;
+  // Per item k: wait for its DMA, barrier, finish the epilogue of item k-1
+  // (its partial sums were written before this barrier), read item k's slot
+  // into registers, barrier (the slot is free), refill the slot with item
+  // k+NB, and only then multiply.  A run of items ends where the (expert,
+  // pass) changes; the A operands are then reloaded (waiting for everything
+  // in flight).
   int k = 0;
   bool pend = false;                    // an item waits for its epilogue
   int p_n = 0, p_rr = 0, p_cnt = 0;     // that item's column, row, rows, first row
   int64_t p_row0 = 0;
   uint32_t p_braw = 0;
   while (true) {
-    // steps until the next group change of either team
-    const int mine_left = k < tn ? min(tn - k, S - ci.s) : nsteps - k;
-    int seg_end = k + mine_left;
-    if constexpr (TEAMS == 2) {
-      // (LDS-only barriers: __syncthreads() would also wait for every DMA in flight)
-      if (lane == 0 && wave == 0) sSeg[team] = mine_left;
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-      asm volatile("s_barrier" ::: "memory");
-      seg_end = k + min(sSeg[0], sSeg[1]);
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      asm volatile("s_barrier" ::: "memory");
-    }
+    const int seg_end = k + min(n_items - k, S - ci.s);
     for (; k < seg_end; ++k) {
-      const bool act = k < tn;
       const int slot = k % NB;
       const uint32_t sb = ring0 + (uint32_t)(slot * C::SLOT);
-      if (act) wait_tiles_ahead<NP, NB - 1>(min(NB - 1, tn - 1 - k));
+      wait_tiles_ahead<DPI, NB - 1>(min(NB - 1, n_items - 1 - k));
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's partial sums are written
       asm volatile("s_barrier" ::: "memory");
       if (pend) ps_epilogue<EPI>(a, tred, lane, wave, col, p_braw, p_n, p_rr, p_cnt, p_row0);
@@ -1260,7 +1242,7 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
       u32x4_t q[NP];
       uint32_t sc[NP];
       uint32_t braw = 0;
-      if (act) {
+      if (live) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
           q[p] = lds_read_b128(sb + p * C::PART + boff);
@@ -1275,11 +1257,11 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
       // every wave has its operands (and is done with the partial sums of
       // the previous item): the slot and the partial-sum buffer are free
       asm volatile("s_barrier" ::: "memory");
-      if (act) {
-        if (k + NB < tn) {
-          ps_issue<G>(a, tring + slot * C::SLOT, ii.e, ii.s * 16, wave, lane, eb);
-          ps_next(ii, sHit, S, nhit);
-        }
+      if (k + NB < n_items) {
+        ps_issue<G, RG>(a, ring + slot * C::SLOT, ii.e, ii.s * 16, rg, wave, lane, eb);
+        ps_next<ROWS>(ii, sHit, S, nhit);
+      }
+      if (live) {
         // groups past G meet zero activations (their slots hold scales)
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1294,25 +1276,26 @@ __global__ __launch_bounds__(256 * TEAMS, 3 - TEAMS) void moe_stream_persist_ker
         pend = true;
         p_braw = braw;
         p_n = ci.s * 16 + col;
-        p_rr = ci.pass * 16 + 4 * c + wave;
+        p_rr = ci.pass * ROWS + 16 * rg + 4 * c + wave;
         p_cnt = ci.cnt;
         p_row0 = row0;
-        ++ci.s;
       }
+      ++ci.s;
     }
-    if (k >= nsteps) break;
-    // this team's group changed: reload its A operands
-    if (k < tn && ci.s == S) {
-      ci.s = S - 1;
-      ps_next(ci, sHit, S, nhit);
-      row0 = __builtin_amdgcn_readfirstlane(sRow0[ci.h]);
+    if (k >= n_items) break;
+    // the (expert, pass) changed: reload the A operands
+    ci.s = S - 1;
+    ps_next<ROWS>(ci, sHit, S, nhit);
+    row0 = __builtin_amdgcn_readfirstlane(sRow0[ci.h]);
+    live = ci.pass * ROWS + 16 * rg < ci.cnt;
+    if (live) {
       u32x4_t raw[NP][4];
-      ps_load_a_raw<G>(a, row0, ci.cnt, ci.pass, col, c, wave, raw);
+      ps_load_a_raw<G>(a, row0, ci.cnt, ci.pass * ROWS + 16 * rg, col, c, wave, raw);
       wait_vmcnt<0>();
       ps_quant_a<G>(raw, c, wave, ah, al, sah, sal);
     }
   }
-  // the last items' epilogues
+  // the last item's epilogue
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   asm volatile("s_barrier" ::: "memory");
   if (pend) ps_epilogue<EPI>(a, tred, lane, wave, col, p_braw, p_n, p_rr, p_cnt, p_row0);
@@ -1829,7 +1812,9 @@ struct MxCfg {
   static constexpr int STAGE = B_OFF + B_BYTES;
   static constexpr int A_DMA = 16 / W;                // A instructions per wave per stage
   static constexpr int B_DMA = BN / 32 / W;           // B instructions per wave per stage
-  static constexpr int DMA_PER_TILE = A_DMA + 1 + B_DMA;
+  // instructions per wave per stage; a wave whose A rows all lie past the
+  // tile's rows (AL = false) leaves them and their scales out
+  static constexpr int dma_per_tile(bool al) { return (al ? A_DMA + 1 : 0) + B_DMA; }
   static constexpr int EPI_LDS = epi_lds_bytes(2, NB);  // per-wave epilogue staging bytes
 };
 
@@ -1876,18 +1861,20 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
 // the B codes.  A device function rather than a lambda: HIP-Clang does not
 // emit the host-side handle of these kernel templates when their bodies call
 // a capturing lambda.
-template <class C, int MX_NS>
+template <class C, int MX_NS, bool AL>
 __device__ __forceinline__ void mx_issue(uint8_t* smem, int kt, const MxLane<C>& l) {
   uint8_t* st = smem + (kt % MX_NS) * C::STAGE;
   const int wave = l.wave;
-  const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
+  if constexpr (AL) {
+    const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
 #pragma unroll
-  for (int j = 0; j < C::A_DMA; ++j) {
-    const uint8_t* src = a + l.aoff_src[j];
-    __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + (C::A_DMA * wave + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < C::A_DMA; ++j) {
+      const uint8_t* src = a + l.aoff_src[j];
+      __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + (C::A_DMA * wave + j) * 1024), 16, 0, 0);
+    }
+    const uint8_t* ssrc = uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src;
+    __builtin_amdgcn_global_load_lds(ssrc, (lds_void*)(st + MX_A_BYTES + 256 * wave), 4, 0, 0);
   }
-  const uint8_t* ssrc = uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src;
-  __builtin_amdgcn_global_load_lds(ssrc, (lds_void*)(st + MX_A_BYTES + 256 * wave), 4, 0, 0);
   const uint8_t* b = uniform_ptr(l.bbase + (int64_t)kt * l.bkt);
 #pragma unroll
   for (int h = 0; h < C::B_DMA; ++h) {
@@ -1972,7 +1959,7 @@ __device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F
 // reads of "step kt+1" fetch a stale stage (in bounds, never used) and the
 // wait and barrier are no-ops, so every wave passes KT + 1 barriers whatever
 // NMB is.
-template <class C, int MX_NS, int NMB, int ISSUE>
+template <class C, int MX_NS, int NMB, bool AL, int ISSUE>
 __device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][C::NBLK], MxB<C::NBLK>& bc, MxB<C::NBLK>& bn,
                                               MxA& a0, MxA& a1, int kt, int KT, uint8_t* smem, const MxLane<C>& l) {
   constexpr int NB = C::NBLK;
@@ -1989,15 +1976,15 @@ __device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][C::NBLK], MxB<C
   // step kt+1 has landed for every wave, and every wave is done reading
   // stage kt (its A1 reads waited for here)
   if constexpr (ISSUE == 1)
-    wait_vmcnt<(MX_NS - 2) * C::DMA_PER_TILE>();
+    wait_vmcnt<(MX_NS - 2) * C::dma_per_tile(AL)>();
   else
-    wait_tiles_ahead<C::DMA_PER_TILE, MX_NS - 2>(min(MX_NS - 2, KT - 2 - kt));
+    wait_tiles_ahead<C::dma_per_tile(AL), MX_NS - 2>(min(MX_NS - 2, KT - 2 - kt));
   wait_lgkm0();
   asm volatile("s_barrier" ::: "memory");
   if constexpr (ISSUE == 1)
-    mx_issue<C, MX_NS>(smem, kt + MX_NS, l);
+    mx_issue<C, MX_NS, AL>(smem, kt + MX_NS, l);
   else if (kt + MX_NS < KT)
-    mx_issue<C, MX_NS>(smem, kt + MX_NS, l);
+    mx_issue<C, MX_NS, AL>(smem, kt + MX_NS, l);
   if constexpr (NMB > 0) {
     const uint8_t* sn = smem + ((kt + 1) % MX_NS) * C::STAGE;
     mx_read_b(bn, sn, l.boff, l.sb_row, l.G, min(kt + 1, KT - 1));
@@ -2013,11 +2000,11 @@ __device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][C::NBLK], MxB<C
 // that issue a later stage's DMA first (ISSUE = 1, no branch), then the
 // last few with a run-time test (ISSUE = 0).  Ends with every DMA and LDS
 // read complete.
-template <class C, int MX_NS, int NMB>
+template <class C, int MX_NS, int NMB, bool AL>
 __device__ __forceinline__ void mx_kloop(f32x16_t (&acc)[2][C::NBLK], int KT, uint8_t* smem, const MxLane<C>& l) {
   for (int i = 0; i < MX_NS; ++i)
-    if (i < KT) mx_issue<C, MX_NS>(smem, i, l);
-  wait_tiles_ahead<C::DMA_PER_TILE, MX_NS - 1>(min(MX_NS - 1, KT - 1));
+    if (i < KT) mx_issue<C, MX_NS, AL>(smem, i, l);
+  wait_tiles_ahead<C::dma_per_tile(AL), MX_NS - 1>(min(MX_NS - 1, KT - 1));
   asm volatile("s_barrier" ::: "memory");
   MxB<C::NBLK> b0, b1;
   MxA a0, a1;
@@ -2027,15 +2014,120 @@ __device__ __forceinline__ void mx_kloop(f32x16_t (&acc)[2][C::NBLK], int KT, ui
   }
   int kt = 0;
   for (; kt + 1 < KT - MX_NS; kt += 2) {
-    mx_split_step<C, MX_NS, NMB, 1>(acc, b0, b1, a0, a1, kt, KT, smem, l);
-    mx_split_step<C, MX_NS, NMB, 1>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
+    mx_split_step<C, MX_NS, NMB, AL, 1>(acc, b0, b1, a0, a1, kt, KT, smem, l);
+    mx_split_step<C, MX_NS, NMB, AL, 1>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
   }
   for (; kt < KT; kt += 2) {
-    mx_split_step<C, MX_NS, NMB, 0>(acc, b0, b1, a0, a1, kt, KT, smem, l);
-    if (kt + 1 < KT) mx_split_step<C, MX_NS, NMB, 0>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
+    mx_split_step<C, MX_NS, NMB, AL, 0>(acc, b0, b1, a0, a1, kt, KT, smem, l);
+    if (kt + 1 < KT) mx_split_step<C, MX_NS, NMB, AL, 0>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
   }
   wait_vmcnt<0>();
   wait_lgkm0();
+}
+
+// --- thin tiles --------------------------------------------------------------
+// A tile of at most 64 live rows (one or two row blocks, MB) has little to
+// multiply and streams weights: in the 2 x 2 wave grid half the waves idle
+// and two stages of mostly dead A rows keep 25 KiB in flight.  Here every wave
+// takes all MB row blocks against 64 of the 256 weight rows, and stages of
+// only the live rows' A (MB x 4 KiB codes, one 256-byte slot of scale dwords
+// that all waves write alike) and B share the same LDS: four stages at MB = 1,
+// three at MB = 2.  The MFMAs of one output go in the k order of the 2 x 2
+// grid (each k-step's hi, then lo), so a row's result does not depend on
+// which form its tile takes.
+template <int MB>
+struct MxThin {
+  static constexpr int NS = MB == 1 ? 4 : 3;
+  static constexpr int AS_OFF = MB * 4096;
+  static constexpr int B_OFF = AS_OFF + 256;
+  static constexpr int STAGE = B_OFF + 256 * 32;
+  static constexpr int PER = MB + 1 + 2;  // DMA instructions per wave per stage
+};
+
+template <class C, int MB>
+__device__ __forceinline__ void mx_thin_issue(uint8_t* smem, int kt, const MxLane<C>& l) {
+  using TH = MxThin<MB>;
+  uint8_t* st = smem + (kt % TH::NS) * TH::STAGE;
+  const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
+#pragma unroll
+  for (int j = 0; j < MB; ++j)
+    __builtin_amdgcn_global_load_lds(a + l.aoff_src[j], (lds_void*)(st + (MB * l.wave + j) * 1024), 16, 0, 0);
+  __builtin_amdgcn_global_load_lds(uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src, (lds_void*)(st + TH::AS_OFF), 4,
+                                   0, 0);
+  const uint8_t* b = uniform_ptr(l.bbase + (int64_t)kt * l.bkt);
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    __builtin_amdgcn_global_load_lds(b + l.boff_src[h], (lds_void*)(st + TH::B_OFF + (2 * l.wave + h) * 1024), 16, 0, 0);
+}
+
+// `mul`: the wave's weight rows are not all past N.
+template <class C, int MB>
+__device__ __forceinline__ void mx_thin_kloop(f32x16_t (&acc)[MB][2], bool mul, int KT, uint8_t* smem,
+                                              const MxLane<C>& l) {
+  using TH = MxThin<MB>;
+  for (int i = 0; i < TH::NS - 1; ++i)
+    if (i < KT) mx_thin_issue<C, MB>(smem, i, l);
+  for (int kt = 0; kt < KT; ++kt) {
+    // stage kt has landed for every wave, and every wave is done reading
+    // stage kt - 1, which takes step kt + NS - 1
+    wait_tiles_ahead<TH::PER, TH::NS - 2>(min(TH::NS - 2, KT - 1 - kt));
+    wait_lgkm0();
+    asm volatile("s_barrier" ::: "memory");
+    if (kt + TH::NS - 1 < KT) mx_thin_issue<C, MB>(smem, kt + TH::NS - 1, l);
+    if (!mul) continue;
+    const uint8_t* st = smem + (kt % TH::NS) * TH::STAGE;
+    MxB<2> b;
+    mx_read_b(b, st, l.boff, l.sb_row, l.G, kt);
+    MxA x[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+      mx_read_a(x[mb], st + mb * 4096, st + l.asoff + mb * 128, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) mx_mfma_row(acc[mb], x[mb], b);
+  }
+  wait_vmcnt<0>();
+  wait_lgkm0();
+}
+
+// The whole thin tile: `rows` (at most 32 MB) sorted rows from m0 against
+// weight rows n0 .. n0 + 255.  l holds what both forms share.
+template <int EPI, class C, int MB>
+__device__ __forceinline__ void mx_thin_tile(const GemmArgs& a, MxLane<C>& l, int e, int m0, int rows, int n0,
+                                             const uint8_t* sbs, uint8_t* smem) {
+  static_assert(C::W == 4 && C::BN == 256, "four waves of 64 weight rows");
+  const int l32 = l.lane & 31;
+  const int lh = l.lane >> 5;
+#pragma unroll
+  for (int j = 0; j < MB; ++j) {
+    const int r = 8 * (MB * l.wave + j) + (l.lane >> 3);
+    l.aoff_src[j] = (uint32_t)(r * 128 + (((l.lane & 7) ^ ((r >> 1) & 7)) * 16));
+  }
+  l.soff_src = (uint32_t)((l.lane % (32 * MB)) * 4);
+  float bias[2];
+  int bq[2];
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb) {
+    bq[nb] = l.wave * 64 + nb * 32 + l32;
+    bias[nb] = n0 + bq[nb] < a.N ? bias_at(a.bias, a.bias_dtype, (int64_t)e * a.N + n0 + bq[nb]) : 0.f;
+  }
+  const int rsw = (l32 >> 1) & 7;
+  l.aoff0 = (uint32_t)(l32 * 128 + ((lh ^ rsw) * 16));
+  l.aoff1 = (uint32_t)(l32 * 128 + (((2 + lh) ^ rsw) * 16));
+  l.aoff2 = (uint32_t)(l32 * 128 + (((4 + lh) ^ rsw) * 16));
+  l.aoff3 = (uint32_t)(l32 * 128 + (((6 + lh) ^ rsw) * 16));
+  l.asoff = (uint32_t)(MxThin<MB>::AS_OFF + l32 * 4 + lh);
+  l.boff = (uint32_t)(MxThin<MB>::B_OFF + bq[0] * 32 + ((lh ^ ((bq[0] >> 3) & 1)) * 16));
+  l.sb_row = sbs + bq[0] * l.G + lh;
+  f32x16_t acc[MB][2];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  mx_thin_kloop<C, MB>(acc, n0 + l.wave * 64 < a.N, a.K / MX_BK, smem, l);
+  __syncthreads();
+  epilogue_staged<EPI, MB, 2>(a, acc, bias, m0, 0, rows, n0 + l.wave * 64, smem + l.wave * epi_lds_bytes(MB, 2), l.lane);
 }
 
 template <int EPI, int MX_NS, bool SB16, int WM, int WN, int NB>
@@ -2047,6 +2139,9 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   static_assert(W == 4 || W == 8, "wave grid");
   static_assert(C::B_DMA * W * 32 == C::BN, "B stage split over the waves");
   static_assert(32 % C::AS_ROWS == 0, "whole scale slots per row block");
+  static_assert(MxThin<1>::NS * MxThin<1>::STAGE <= MX_NS * C::STAGE &&
+                    MxThin<2>::NS * MxThin<2>::STAGE <= MX_NS * C::STAGE,
+                "the thin tiles' stages fit below the B scales");
   constexpr int BN = C::BN;
   extern __shared__ __align__(1024) uint8_t smem[];
   const int L = xcd_tile_index(*a.num_tiles * a.n_tiles_n);
@@ -2104,6 +2199,14 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   l.lane = lane;
   l.G = G;
 
+  if (rows <= 64) {
+    if (rows <= 32)
+      mx_thin_tile<EPI, C, 1>(a, l, e, m0, rows, n0, sbs, smem);
+    else
+      mx_thin_tile<EPI, C, 2>(a, l, e, m0, rows, n0, sbs, smem);
+    return;
+  }
+
   // this lane's B rows (one per 32-column block) and their bias
   int bq[NB];
   float bias[NB];
@@ -2143,12 +2246,19 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   // whose weight rows all lie past N (in the last column tile: half of it at
   // gate_up's N = 5760, and at down's N = 2880).
   const int nmb = n0 + wn * C::WCOLS < a.N ? min(2, max(0, (rows - 64 * wm + 31) / 32)) : 0;
+  // The wave's share of the A stage is left out when it lies past the tile's
+  // rows: a tile of one 32-row block then streams 12 KiB a step, not 24.
+  const bool al = 8 * C::A_DMA * wave < rows;
   if (nmb == 2)
-    mx_kloop<C, MX_NS, 2>(acc, KT, smem, l);
+    mx_kloop<C, MX_NS, 2, true>(acc, KT, smem, l);
+  else if (nmb == 1 && al)
+    mx_kloop<C, MX_NS, 1, true>(acc, KT, smem, l);
   else if (nmb == 1)
-    mx_kloop<C, MX_NS, 1>(acc, KT, smem, l);
+    mx_kloop<C, MX_NS, 1, false>(acc, KT, smem, l);
+  else if (al)
+    mx_kloop<C, MX_NS, 0, true>(acc, KT, smem, l);
   else
-    mx_kloop<C, MX_NS, 0>(acc, KT, smem, l);
+    mx_kloop<C, MX_NS, 0, false>(acc, KT, smem, l);
 
   // epilogue through LDS: the stage buffers are free once every wave is done
   __syncthreads();
@@ -2644,7 +2754,7 @@ static int allow_big_lds(const void* fn, int kind, int epi, int bytes = 160 * 10
     set_error("no current HIP device");
     return BSA_EHIP;
   }
-  // kinds: 1-3 packed-weight backward kernel, 4-5 tiled kernel, 6 persistent
+  // kinds: 1-3 packed-weight backward kernel, 4-5 tiled kernel, 6-7 persistent
   // decode kernel, 8-15 MX kernel configurations
   static bool allowed[64][16][8];
   if (!allowed[dev][kind][epi]) {
@@ -2741,7 +2851,7 @@ static int cu_count() {
 // kernel (else the one-workgroup-per-slice stream kernel).
 static bool persist_ok(const GemmArgs& a, int64_t P) {
   auto al16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-  return a.K == 2880 && a.N % 16 == 0 && a.E <= 256 * PS_TEAMS && al16(a.Bq) && al16(a.Bs) && al16(a.bias) &&
+  return a.K == 2880 && a.N % 16 == 0 && a.E <= 256 && al16(a.Bq) && al16(a.Bs) && al16(a.bias) &&
          al16(a.A) && a.lda % 8 == 0 && P <= (1 << 19) && cu_count() > 0;
 }
 
@@ -2764,6 +2874,24 @@ static int run_dispatch(const int64_t* idx, int64_t P, int E, const Workspace& w
   // the activation buffer, which gate_up overwrites afterwards
   return launch_dispatch(idx, (int)P, E, TL_BM, w.counts, w.offsets, w.row_pair, w.pair_pos, w.tiles,
                          w.num_tiles, reinterpret_cast<int*>(w.act), st);
+}
+
+// Row groups (16-row blocks sharing one read of the weights) of the
+// persistent kernel: two once experts commonly hold more than 16 rows.  120b
+// layer, one against two (unevenly hit experts): 64 tokens 199 / 218 us, 128
+// 245 / 252, 256 338 / 325, 512 514 / 420.  (Four waves' operands of 32 rows do
+// not fit a wave's registers, so two groups take 512 threads and the CU's
+// whole ring, which the smaller batches, with fewer rows to share, pay for.)
+static int ps_row_groups(int64_t P, int64_t E) { return P > 6 * E ? 2 : 1; }
+
+template <int EPI, int RG>
+static int launch_persist(const GemmArgs& a, int cus, hipStream_t st) {
+  constexpr int ring = PS_NB * RG * PsCfg<90>::SLOT;
+  int rc = allow_big_lds(reinterpret_cast<const void*>(moe_stream_persist_kernel<EPI, 90, RG>), 5 + RG, EPI, ring);
+  if (rc) return rc;
+  hipLaunchKernelGGL((moe_stream_persist_kernel<EPI, 90, RG>), dim3((unsigned)(cus * 2 / RG)), dim3(256 * RG), ring, st, a);
+  BSA_LAUNCH_CHECK("grouped GEMM launch");
+  return BSA_OK;
 }
 
 // `pending` (non-null for the first GEMM of a forward whose dispatch has not
@@ -2795,14 +2923,8 @@ static int launch_gemm(const GemmArgs& a, int path, int64_t P, hipStream_t st,
       int rc = run_dispatch(pending->idx, P, a.E, *pending->w, st);
       if (rc) return rc;
     }
-    constexpr int ring = PS_TEAMS * PS_TEAM_NB * PsCfg<90>::SLOT;
-    const void* fn = reinterpret_cast<const void*>(moe_stream_persist_kernel<EPI, 90, PS_TEAMS>);
-    int rc = allow_big_lds(fn, 6, EPI, ring);
-    if (rc) return rc;
-    hipLaunchKernelGGL((moe_stream_persist_kernel<EPI, 90, PS_TEAMS>), dim3((unsigned)(cus * (3 - PS_TEAMS))),
-                       dim3(256 * PS_TEAMS), ring, st, b);
-    BSA_LAUNCH_CHECK("grouped GEMM launch");
-    return BSA_OK;
+    if (ps_row_groups(P, a.E) == 2) return launch_persist<EPI, 2>(b, cus, st);
+    return launch_persist<EPI, 1>(b, cus, st);
   }
   if (pending) {
     int rc = run_dispatch(pending->idx, P, a.E, *pending->w, st);

@@ -188,3 +188,32 @@ def test_mx_concentrated_and_duplicate_routing(device):
         got = kernels.moe_experts_forward(t["hidden"], ix, w, *args, path="mx")
         want = oracle.experts_ref(t["hidden"].cpu(), ix.cpu(), w.cpu().float(), *cpu_args)
         assert_layer_close(got, want, f"MX {what}", absolute=True)
+
+
+@pytest.mark.parametrize("H,I", [(64, 64), (128, 192), (448, 320), (832, 1600), (2880, 2880)])
+def test_mx_tile_row_edges(device, H, I):
+    """Experts whose row counts sit at the edges of the 32-row blocks, of the thin tiles and of the
+    128-row tiles, for k loops of one to 45 steps: against the float32 oracle, and every token's row bit for bit
+    the one it gets in a batch of its own (whichever form its tile takes there)."""
+    counts = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 0, 161]
+    E, T = len(counts), sum(counts)
+    t, _, _ = _layer(E, 1, H, I, T, seed=H + I, device=device)
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(2))
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[order].reshape(T, 1).to(device)
+    w = torch.rand(T, 1, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(device)
+    announce(f"mx tile edges H={H} I={I}")
+    got = kernels.moe_experts_forward(t["hidden"], idx, w, *expert_args(t), path="mx")
+    kp = [x if i not in (0, 3) or H % 64 or I % 64 or (H // 32) % 2 or (I // 32) % 2 else kernels.to_kpair(x)
+          for i, x in enumerate(expert_args(t))]
+    got_kp = kernels.moe_experts_forward(t["hidden"], idx, w, *kp, path="mx")
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), got_kp.view(torch.int16))
+    args = [a.cpu() for a in expert_args(t)]
+    want = oracle.experts_ref(t["hidden"].cpu(), idx.cpu(), w.cpu().float(), *args)
+    assert_layer_close(got, want, f"mx tile edges {H} {I}")
+    for e in range(E):
+        rows = (idx[:, 0] == e).nonzero()[:1, 0]
+        if not len(rows):
+            continue
+        one = kernels.moe_experts_forward(t["hidden"][rows], idx[rows], w[rows], *expert_args(t), path="mx")
+        assert torch.equal(one.view(torch.int16), got[rows].view(torch.int16)), f"expert {e}"

@@ -136,3 +136,29 @@ def test_persistent_f16_or_no_bias_vs_oracle(device, bias):
     got = kernels.moe_experts_forward(t["hidden"], idx, w, *args, path="stream")
     want = oracle.experts_ref(t["hidden"].cpu(), idx.cpu(), w.cpu().float(), *ref_args)
     assert_layer_close(got, want, f"bias {bias}", absolute=True)
+
+
+@pytest.mark.parametrize("rows", [(1, 15), (16, 17), (32, 33), (64, 65), (95, 100)])
+def test_persistent_two_row_groups_edges(device, rows):
+    """Batches with two row groups per workgroup (32-row passes): experts at the edges of
+    a group and of a pass, against the part kernel and the oracle.  A token's row does
+    not depend on the batch: the same tokens one by one (one row group) give the same bits."""
+    E, k = 8, 1
+    counts = [rows[0], rows[1], 0, 32, 16, 1, 48, 31]
+    T = sum(counts)
+    t = synthetic.moe_layer(synthetic.MoEShape(E, k, 2880, 2880, T), seed=61, scale_lo=116, scale_hi=120,
+                            device=device)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(
+        T, generator=torch.Generator().manual_seed(1))].reshape(T, k).to(device)
+    w = torch.full((T, k), 0.5, dtype=torch.bfloat16, device=device)
+    assert T * k > 6 * E
+    announce(f"persistent kernel, two row groups, counts {counts}")
+    persist, parts = _both_kernels(t, idx, w)
+    _agree(persist, parts, f"counts {counts}")
+    tokens = torch.arange(0, T, 23)
+    want = oracle_tokens(t, idx.cpu(), w.cpu(), tokens)
+    assert_layer_close(persist.cpu()[tokens], want, f"counts {counts}", absolute=True)
+    for i in tokens[:4].tolist():
+        one = kernels.moe_experts_forward(t["hidden"][i:i + 1], idx[i:i + 1], w[i:i + 1], *expert_args(t),
+                                          path="stream")
+        assert torch.equal(one.view(torch.int16), persist[i:i + 1].view(torch.int16))
