@@ -1789,61 +1789,64 @@ __device__ __forceinline__ int64_t tile_src_row(const GemmArgs& a, int m0, int r
   return a.row_pair ? (int64_t)(a.row_pair[pos] / a.topk) : pos;
 }
 
-// Per-configuration sizes: a 2 x WN wave grid, wave (wm, wn) owning the two
-// row blocks 2wm, 2wm+1 and NB column blocks of 32 x 32 (rows 64*wm ..,
-// weight rows 32*NB*wn .. of the tile); BN = 32 * NB * WN weight rows per
-// tile.  A stage holds the A codes (16 KiB), the A scale dwords and the B
-// codes.  The scale dwords sit in one 256-byte slot per wave: its AS_ROWS
-// rows, then padding that the wave's other lanes fill with copies, so the
-// scale DMA is a whole-wave instruction (no divergent branch in the k loop).
-// The B scales of the tile's weight rows are loaded once per tile (per-stage
-// loads of their two bytes per row measured slower: one request per row).
-template <int WN, int NB>
-struct MxCfg {
-  static constexpr int W = 2 * WN;                    // waves
-  static constexpr int NBLK = NB;
-  static constexpr int WCOLS = 32 * NB;
-  static constexpr int BN = WCOLS * WN;
-  static constexpr int B_BYTES = BN * 32;
-  static constexpr int AS_ROWS = MX_BM / W;           // A scale rows per wave (one dword each)
-  static constexpr int AS_BYTES = W * 256;
-  static constexpr int AS_BLOCK = 32 / AS_ROWS * 256; // slot bytes per 32-row block
-  static constexpr int B_OFF = MX_A_BYTES + AS_BYTES;
-  static constexpr int STAGE = B_OFF + B_BYTES;
-  static constexpr int A_DMA = 16 / W;                // A instructions per wave per stage
-  static constexpr int B_DMA = BN / 32 / W;           // B instructions per wave per stage
-  // instructions per wave per stage; a wave whose A rows all lie past the
-  // tile's rows (AL = false) leaves them and their scales out
-  static constexpr int dma_per_tile(bool al) { return (al ? A_DMA + 1 : 0) + B_DMA; }
-  static constexpr int EPI_LDS = epi_lds_bytes(2, NB);  // per-wave epilogue staging bytes
-};
-
-// Dynamic LDS bytes of moe_mx_kernel with ns stages: the stages and the B
-// scales.
-template <class C>
-inline size_t mx_smem_bytes(int ns, int K) {
-  return (size_t)ns * C::STAGE + (size_t)C::BN * (K / 32);
-}
-
-// Workgroups per CU (the launch bound); two hide each other's barrier and
-// DMA waits, and the 2 x 2 wave grid's stages and B scales fit both in LDS.
-#ifndef BSA_MX_WG_PER_CU
-#define BSA_MX_WG_PER_CU 2
-#endif
+// A 2 x 2 wave grid, wave (wm, wn) owning the two row blocks 2wm, 2wm+1 and
+// four column blocks of 32 x 32 (rows 64*wm .., weight rows 128*wn .. of the
+// tile): 256 weight rows per tile.
+//
+// LDS (80 KiB, two workgroups per CU):
+//  * two A stages of one 64-k step: codes (16 KiB) and scale dwords, the latter
+//    in one 256-byte slot per wave (its 32 rows, then copies, so that the
+//    scale DMA is a whole-wave instruction);
+//  * two B stages of a PAIR of steps, 1 KiB per 16 weight rows (one DMA
+//    instruction).  Checkpoint layout: [row][64 B], 16-byte group g of row q in
+//    position g ^ ((q >> 2) & 3).  A row's 64 bytes are one request of the DMA
+//    where two steps' 32 bytes were two: the address path, not the bytes, is
+//    what the weight stream costs there (120b layer, one step's 32 bytes against
+//    two steps' 64: 256 tokens on this kernel 487 -> 423 us, 1000 668 -> 592, 2000 776
+//    -> 694, 8192 1706 -> 1662).  K-pair layout: [step][row][32
+//    B] (two runs of 512 bytes, as in memory), half g of row q in position g ^
+//    ((q >> 3) & 1).  Either way the 16 rows one ds_read_b128 pass serves sit
+//    in 16 different bank groups, and the pair's two steps are bpar apart;
+//  * two chunks of B scales: the bytes of 12 steps (24 per row) in seven dwords
+//    per row from the dword that holds the first (a row's bytes start 0 or 2
+//    bytes into it).  An odd dword stride keeps the byte reads of 32 rows free of
+//    conflicts, and the whole tile's scales (22.5 KiB at K = 2880) would not
+//    leave room for the B pairs.
+constexpr int MX_W = 4;                                // waves
+constexpr int MX_NB = 4;                               // column blocks per wave
+constexpr int MX_WCOLS = 32 * MX_NB;
+constexpr int MX_BN = 2 * MX_WCOLS;
+constexpr int MX_A_STAGE = MX_A_BYTES + MX_W * 256;
+constexpr int MX_B_PAIR = MX_BN * 64;
+constexpr int MX_SC_STEPS = 12;                        // steps per scale chunk
+constexpr int MX_SC_ROW = 28;                          // LDS bytes per row of a chunk
+constexpr int MX_SC_CHUNK = MX_BN * MX_SC_ROW;
+constexpr int MX_B_OFF = 2 * MX_A_STAGE;
+constexpr int MX_SC_OFF = MX_B_OFF + 2 * MX_B_PAIR;
+constexpr int MX_SMEM = MX_SC_OFF + 2 * MX_SC_CHUNK;
+constexpr int MX_A_DMA = 4;                            // A code instructions per wave per step
+constexpr int MX_B_DMA = 4;                            // B instructions per wave per pair
+constexpr int MX_SC_DMA = MX_SC_CHUNK / 4 / 64 / MX_W; // scale instructions per wave per chunk
+static_assert(MX_SMEM <= 80 * 1024, "two workgroups per CU");
+static_assert(MX_SC_DMA * 64 * MX_W * 4 == MX_SC_CHUNK, "whole scale instructions");
+static_assert(2 * MX_SC_STEPS + 2 <= MX_SC_ROW && MX_SC_STEPS % 2 == 0, "a chunk row covers its bytes");
 
 // Per-lane DMA sources (workgroup-uniform bases plus 32-bit per-lane
 // offsets) and LDS read offsets of one tile, set up once.
-template <class C>
 struct MxLane {
   const uint8_t* abase;  // the tile's A codes, k-tile 0
   const uint8_t* sbase;  // the tile's A scale dwords, k-tile 0
   const uint8_t* bbase;  // the expert's packed weights
-  uint32_t aoff_src[C::A_DMA];
+  const uint8_t* bs;     // the dword of the weight scales holding the tile's first
+  uint32_t aoff_src[MX_A_DMA];
   uint32_t soff_src;
-  uint32_t boff_src[C::B_DMA];
+  uint32_t boff_src[MX_B_DMA];
   int64_t lda_kt, lds_kt;
-  int bkt, wave, lane, G;
-  uint32_t aoff0, aoff1, aoff2, aoff3, asoff, boff;
+  int bs_shift;          // scale bytes of the tile's first row before its first dword's
+  int bs_last;           // offset from there of the last dword of the tensor (or far past the tile)
+  int bs_rows;           // weight rows of the tile
+  int bpair, bback, KT, wave, lane, G;
+  uint32_t aoff0, aoff1, aoff2, aoff3, asoff, boff, bpar;
   const uint8_t* sb_row;
 };
 
@@ -1857,38 +1860,64 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
   return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
 }
 
-// Step kt's DMA into stage kt % MX_NS: the A codes, the A scale slot and
-// the B codes.  A device function rather than a lambda: HIP-Clang does not
-// emit the host-side handle of these kernel templates when their bodies call
-// a capturing lambda.
-template <class C, int MX_NS, bool AL>
-__device__ __forceinline__ void mx_issue(uint8_t* smem, int kt, const MxLane<C>& l) {
-  uint8_t* st = smem + (kt % MX_NS) * C::STAGE;
-  const int wave = l.wave;
+// The DMA pieces of a tile.  Device functions rather than lambdas: HIP-Clang
+// does not emit the host-side handle of these kernel templates when their
+// bodies call a capturing lambda.
+// A of step kt into stage kt % 2 (AL: the wave has live A rows).
+template <bool AL>
+__device__ __forceinline__ void mx_issue_a(uint8_t* smem, int kt, const MxLane& l) {
   if constexpr (AL) {
+    uint8_t* st = smem + (kt & 1) * MX_A_STAGE;
     const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
 #pragma unroll
-    for (int j = 0; j < C::A_DMA; ++j) {
+    for (int j = 0; j < MX_A_DMA; ++j) {
       const uint8_t* src = a + l.aoff_src[j];
-      __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + (C::A_DMA * wave + j) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + (MX_A_DMA * l.wave + j) * 1024), 16, 0, 0);
     }
     const uint8_t* ssrc = uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src;
-    __builtin_amdgcn_global_load_lds(ssrc, (lds_void*)(st + MX_A_BYTES + 256 * wave), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds(ssrc, (lds_void*)(st + MX_A_BYTES + 256 * l.wave), 4, 0, 0);
   }
-  const uint8_t* b = uniform_ptr(l.bbase + (int64_t)kt * l.bkt);
+}
+
+// B of the pair of steps 2p, 2p + 1 to st.  In a last pair of one step the
+// lanes of the missing one repeat its partner.
+__device__ __forceinline__ void mx_issue_b(uint8_t* st, int p, const MxLane& l) {
+  const uint8_t* b = uniform_ptr(l.bbase + (int64_t)p * l.bpair);
+  const bool half = 2 * p + 1 >= l.KT;
 #pragma unroll
-  for (int h = 0; h < C::B_DMA; ++h) {
-    const uint8_t* src = b + l.boff_src[h];
-    __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + C::B_OFF + (C::B_DMA * wave + h) * 1024), 16, 0, 0);
+  for (int h = 0; h < MX_B_DMA; ++h) {
+    const uint8_t* src = b + (half ? l.boff_src[h] - l.bback : l.boff_src[h]);
+    __builtin_amdgcn_global_load_lds(src, (lds_void*)(st + (MX_B_DMA * l.wave + h) * 1024), 16, 0, 0);
   }
+}
+
+// B scales of steps 12c .. 12c + 11 into chunk buffer c % 2.  A chunk past K
+// reads whatever follows (never used), dwords past the tensor its last one.
+__device__ __forceinline__ void mx_issue_scales(uint8_t* smem, int c, const MxLane& l) {
+  uint8_t* st = smem + MX_SC_OFF + (c & 1) * MX_SC_CHUNK;
+#pragma unroll
+  for (int j = 0; j < MX_SC_DMA; ++j) {
+    const int i = MX_SC_DMA * l.wave + j;
+    const int x = 64 * i + l.lane;
+    const int row = x / (MX_SC_ROW / 4);
+    const int d = x - row * (MX_SC_ROW / 4);
+    const int o = ((l.bs_shift + min(row, l.bs_rows - 1) * l.G) & ~3) + 2 * MX_SC_STEPS * c + 4 * d;
+    __builtin_amdgcn_global_load_lds(uniform_ptr(l.bs) + (uint32_t)min(o, l.bs_last), (lds_void*)(st + i * 256), 4, 0, 0);
+  }
+}
+
+// Byte offset of step kt's scale pair within a row of the chunk buffers.
+__device__ __forceinline__ int mx_scale_off(int kt) {
+  const int c = kt / MX_SC_STEPS;
+  return (c & 1) * MX_SC_CHUNK + 2 * (kt - c * MX_SC_STEPS);
 }
 
 // --- split-step pipeline ---------------------------------------------------
 // Step kt's MFMAs run in two halves, row block 0 then row block 1, and every
 // LDS read is issued one half ahead of the MFMAs that use it:
-//   read A1(kt) | MFMAs row 0 (B(kt), A0(kt)) | wait for stage kt+1, barrier,
-//   DMA step kt+NS into stage kt, read B(kt+1), A0(kt+1) | MFMAs row 1
-//   (B(kt), A1(kt)).
+//   read A1(kt) | MFMAs row 0 (B(kt), A0(kt)) | wait for A(kt+1), barrier,
+//   DMA of A(kt+2) into stage kt (and on odd steps of the B pair kt+3, kt+4),
+//   read B(kt+1), A0(kt+1) | MFMAs row 1 (B(kt), A1(kt)).
 // So a wave does not wait on its own LDS reads; B alternates between two
 // register sets (row 1 still multiplies B(kt) while B(kt+1) lands), A0 and
 // A1 are overwritten in place once their MFMAs have issued.  The one barrier
@@ -1908,13 +1937,15 @@ struct MxB {
   int sb[NB];
 };
 
+// B(kt) from its pair's stage.
 template <int NB>
-__device__ __forceinline__ void mx_read_b(MxB<NB>& f, const uint8_t* st, uint32_t boff, const uint8_t* sb_row, int G,
-                                          int kt) {
+__device__ __forceinline__ void mx_read_b(MxB<NB>& f, const uint8_t* pair, const MxLane& l, int kt) {
+  const uint8_t* b = pair + (l.boff ^ ((kt & 1) ? l.bpar : 0u));
+  const uint8_t* sb = l.sb_row + mx_scale_off(kt);
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
-    f.sb[nb] = sb_row[nb * 32 * G + 2 * kt];
-    f.b[nb] = *reinterpret_cast<const u32x4_t*>(st + boff + nb * 1024);
+    f.sb[nb] = sb[nb * 32 * MX_SC_ROW];
+    f.b[nb] = *reinterpret_cast<const u32x4_t*>(b + nb * 2048);
   }
 }
 
@@ -1951,43 +1982,46 @@ __device__ __forceinline__ void mx_mfma_row(f32x16_t (&acc)[NB], const MxA& a, c
 // s_waitcnt lgkmcnt(0) (vmcnt and expcnt not waited on)
 __device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
-// Step kt of the split-step pipeline for a wave holding NMB (0..2) row
-// blocks of the tile; bc holds B(kt) and a0 A0(kt) (reads issued), bn
-// receives B(kt+1).  ISSUE: whether this step issues step kt + MX_NS's DMA
-// (decided per call site, so the steady-state steps are one basic block and
-// the first half's MFMAs stay above the barrier).  On the last step the
-// reads of "step kt+1" fetch a stale stage (in bounds, never used) and the
-// wait and barrier are no-ops, so every wave passes KT + 1 barriers whatever
-// NMB is.
-template <class C, int MX_NS, int NMB, bool AL, int ISSUE>
-__device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][C::NBLK], MxB<C::NBLK>& bc, MxB<C::NBLK>& bn,
-                                              MxA& a0, MxA& a1, int kt, int KT, uint8_t* smem, const MxLane<C>& l) {
-  constexpr int NB = C::NBLK;
-  const uint8_t* st = smem + (kt % MX_NS) * C::STAGE;
+// Step kt (of parity ODD) of the split-step pipeline for a wave holding NMB
+// (0..2) row blocks of the tile; bc holds B(kt) and a0 A0(kt) (reads issued),
+// bn receives B(kt+1).  ISSUE 1 and 2: steady-state steps, one basic block
+// each (so the first half's MFMAs stay above the barrier), which fetch
+// without a test; what may stay in flight at the wait are the B pair of the
+// odd step before (an even step) and, with ISSUE 2, the scale chunk issued
+// just before it.  ISSUE 0: the last steps, fetching what is left.  On the last
+// step the reads of "step kt+1" fetch a stale stage (in bounds, never used),
+// so every wave passes KT + 1 barriers whatever NMB is.
+template <int NMB, bool AL, bool ODD, int ISSUE>
+__device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][MX_NB], MxB<MX_NB>& bc, MxB<MX_NB>& bn, MxA& a0,
+                                              MxA& a1, int kt, uint8_t* smem, const MxLane& l) {
+  constexpr int NB = MX_NB;
+  const uint8_t* st = smem + (ODD ? MX_A_STAGE : 0);
   // the first MFMA before the A1 reads: its operands were read a half step
   // ago, and the wait the compiler puts before it then covers only them
   if constexpr (NMB > 0) mx_mfma_row<NB, 0, 1>(acc[0], a0, bc);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (NMB > 1)
-    mx_read_a(a1, st + 32 * 128, st + l.asoff + C::AS_BLOCK, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
+  if constexpr (NMB > 1) mx_read_a(a1, st + 32 * 128, st + l.asoff + 256, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (NMB > 0) mx_mfma_row<NB, 1, 2 * NB>(acc[0], a0, bc);
   __builtin_amdgcn_sched_barrier(0);
-  // step kt+1 has landed for every wave, and every wave is done reading
-  // stage kt (its A1 reads waited for here)
-  if constexpr (ISSUE == 1)
-    wait_vmcnt<(MX_NS - 2) * C::dma_per_tile(AL)>();
+  // A(kt+1) (and its B pair) has landed for every wave, and every wave is
+  // done reading stage kt (its A1 reads waited for here)
+  if constexpr (ISSUE == 0 || ODD)
+    wait_vmcnt<0>();
   else
-    wait_tiles_ahead<C::dma_per_tile(AL), MX_NS - 2>(min(MX_NS - 2, KT - 2 - kt));
+    wait_vmcnt<MX_B_DMA + (ISSUE == 2 ? MX_SC_DMA : 0)>();
   wait_lgkm0();
   asm volatile("s_barrier" ::: "memory");
-  if constexpr (ISSUE == 1)
-    mx_issue<C, MX_NS, AL>(smem, kt + MX_NS, l);
-  else if (kt + MX_NS < KT)
-    mx_issue<C, MX_NS, AL>(smem, kt + MX_NS, l);
+  if constexpr (ISSUE > 0) {
+    mx_issue_a<AL>(smem, kt + 2, l);
+    if constexpr (ODD) mx_issue_b(smem + MX_B_OFF + (((kt + 3) >> 1) & 1) * MX_B_PAIR, (kt + 3) >> 1, l);
+  } else {
+    if (kt + 2 < l.KT) mx_issue_a<AL>(smem, kt + 2, l);
+    if (ODD && kt + 3 < l.KT) mx_issue_b(smem + MX_B_OFF + (((kt + 3) >> 1) & 1) * MX_B_PAIR, (kt + 3) >> 1, l);
+  }
   if constexpr (NMB > 0) {
-    const uint8_t* sn = smem + ((kt + 1) % MX_NS) * C::STAGE;
-    mx_read_b(bn, sn, l.boff, l.sb_row, l.G, min(kt + 1, KT - 1));
+    const uint8_t* sn = smem + (ODD ? 0 : MX_A_STAGE);
+    mx_read_b(bn, smem + MX_B_OFF + (((kt + 1) >> 1) & 1) * MX_B_PAIR, l, kt + 1);
     mx_read_a(a0, sn, sn + l.asoff, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -1995,31 +2029,45 @@ __device__ __forceinline__ void mx_split_step(f32x16_t (&acc)[2][C::NBLK], MxB<C
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// The whole k loop: all MX_NS stages issued up front (after the B scales),
-// then the steps two at a time (B's register sets swap roles): the steps
-// that issue a later stage's DMA first (ISSUE = 1, no branch), then the
-// last few with a run-time test (ISSUE = 0).  Ends with every DMA and LDS
-// read complete.
-template <class C, int MX_NS, int NMB, bool AL>
-__device__ __forceinline__ void mx_kloop(f32x16_t (&acc)[2][C::NBLK], int KT, uint8_t* smem, const MxLane<C>& l) {
-  for (int i = 0; i < MX_NS; ++i)
-    if (i < KT) mx_issue<C, MX_NS, AL>(smem, i, l);
-  wait_tiles_ahead<C::dma_per_tile(AL), MX_NS - 1>(min(MX_NS - 1, KT - 1));
+// The whole k loop: the first scale chunk, two steps of A and two B pairs
+// issued up front, then the steps two at a time (B's register sets swap
+// roles), chunk by chunk of the scales: chunk c + 1 is fetched as chunk c
+// begins, into the buffer of chunk c - 1, which every wave has read by then.
+// Ends with every DMA and LDS read complete.
+template <int NMB, bool AL>
+__device__ __forceinline__ void mx_kloop(f32x16_t (&acc)[2][MX_NB], uint8_t* smem, const MxLane& l) {
+  const int KT = l.KT;
+  mx_issue_scales(smem, 0, l);
+  mx_issue_b(smem + MX_B_OFF, 0, l);
+  mx_issue_a<AL>(smem, 0, l);
+  if (KT > 1) mx_issue_a<AL>(smem, 1, l);
+  if (KT > 2) mx_issue_b(smem + MX_B_OFF + MX_B_PAIR, 1, l);
+  if (KT > 2)
+    wait_vmcnt<(AL ? MX_A_DMA + 1 : 0) + MX_B_DMA>();
+  else
+    wait_vmcnt<0>();
   asm volatile("s_barrier" ::: "memory");
-  MxB<C::NBLK> b0, b1;
+  MxB<MX_NB> b0, b1;
   MxA a0, a1;
   if constexpr (NMB > 0) {
-    mx_read_b(b0, smem, l.boff, l.sb_row, l.G, 0);
+    mx_read_b(b0, smem + MX_B_OFF, l, 0);
     mx_read_a(a0, smem, smem + l.asoff, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
   }
+  // steady state while the pair an odd step fetches (kt + 4, kt + 5) exists
   int kt = 0;
-  for (; kt + 1 < KT - MX_NS; kt += 2) {
-    mx_split_step<C, MX_NS, NMB, AL, 1>(acc, b0, b1, a0, a1, kt, KT, smem, l);
-    mx_split_step<C, MX_NS, NMB, AL, 1>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
+  while (kt + 5 < KT) {
+    mx_issue_scales(smem, kt / MX_SC_STEPS + 1, l);
+    mx_split_step<NMB, AL, false, 2>(acc, b0, b1, a0, a1, kt, smem, l);
+    mx_split_step<NMB, AL, true, 1>(acc, b1, b0, a0, a1, kt + 1, smem, l);
+    const int end = min(kt + MX_SC_STEPS, KT - 5);
+    for (kt += 2; kt < end; kt += 2) {
+      mx_split_step<NMB, AL, false, 1>(acc, b0, b1, a0, a1, kt, smem, l);
+      mx_split_step<NMB, AL, true, 1>(acc, b1, b0, a0, a1, kt + 1, smem, l);
+    }
   }
   for (; kt < KT; kt += 2) {
-    mx_split_step<C, MX_NS, NMB, AL, 0>(acc, b0, b1, a0, a1, kt, KT, smem, l);
-    if (kt + 1 < KT) mx_split_step<C, MX_NS, NMB, AL, 0>(acc, b1, b0, a0, a1, kt + 1, KT, smem, l);
+    mx_split_step<NMB, AL, false, 0>(acc, b0, b1, a0, a1, kt, smem, l);
+    if (kt + 1 < KT) mx_split_step<NMB, AL, true, 0>(acc, b1, b0, a0, a1, kt + 1, smem, l);
   }
   wait_vmcnt<0>();
   wait_lgkm0();
@@ -2027,74 +2075,98 @@ __device__ __forceinline__ void mx_kloop(f32x16_t (&acc)[2][C::NBLK], int KT, ui
 
 // --- thin tiles --------------------------------------------------------------
 // A tile of at most 64 live rows (one or two row blocks, MB) has little to
-// multiply and streams weights: in the 2 x 2 wave grid half the waves idle
-// and two stages of mostly dead A rows keep 25 KiB in flight.  Here every wave
-// takes all MB row blocks against 64 of the 256 weight rows, and stages of
-// only the live rows' A (MB x 4 KiB codes, one 256-byte slot of scale dwords
-// that all waves write alike) and B share the same LDS: four stages at MB = 1,
-// three at MB = 2.  The MFMAs of one output go in the k order of the 2 x 2
-// grid (each k-step's hi, then lo), so a row's result does not depend on
-// which form its tile takes.
+// multiply and streams weights: in the 2 x 2 wave grid half the waves idle.
+// Here every wave takes all MB row blocks against 64 of the 256 weight rows,
+// two steps per barrier.  A stages hold two steps of the live rows only (per
+// step MB x 4 KiB of codes and a 256-byte slot of scale dwords that all waves
+// write alike), which leaves room for three B pairs at MB = 1 (two at MB = 2).
+// The MFMAs of one output go in the k order of the 2 x 2 grid (each step's
+// hi, then lo), so a row's result does not depend on which form its tile takes.
 template <int MB>
 struct MxThin {
-  static constexpr int NS = MB == 1 ? 4 : 3;
-  static constexpr int AS_OFF = MB * 4096;
-  static constexpr int B_OFF = AS_OFF + 256;
-  static constexpr int STAGE = B_OFF + 256 * 32;
-  static constexpr int PER = MB + 1 + 2;  // DMA instructions per wave per stage
+  static constexpr int A_STEP = MB * 4096;
+  static constexpr int A_PAIR = 2 * A_STEP + 512;
+  static constexpr int NBP = MB == 1 ? 3 : 2;   // B pairs
+  static constexpr int B_OFF = 2 * A_PAIR;
+  static_assert(B_OFF + NBP * MX_B_PAIR <= MX_SC_OFF, "the stages fit below the B scales");
 };
 
-template <class C, int MB>
-__device__ __forceinline__ void mx_thin_issue(uint8_t* smem, int kt, const MxLane<C>& l) {
+template <int MB>
+__device__ __forceinline__ void mx_thin_issue_a(uint8_t* smem, int p, const MxLane& l) {
   using TH = MxThin<MB>;
-  uint8_t* st = smem + (kt % TH::NS) * TH::STAGE;
-  const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
+  uint8_t* st = smem + (p & 1) * TH::A_PAIR;
 #pragma unroll
-  for (int j = 0; j < MB; ++j)
-    __builtin_amdgcn_global_load_lds(a + l.aoff_src[j], (lds_void*)(st + (MB * l.wave + j) * 1024), 16, 0, 0);
-  __builtin_amdgcn_global_load_lds(uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src, (lds_void*)(st + TH::AS_OFF), 4,
-                                   0, 0);
-  const uint8_t* b = uniform_ptr(l.bbase + (int64_t)kt * l.bkt);
+  for (int i = 0; i < 2; ++i) {
+    const int kt = min(2 * p + i, l.KT - 1);
+    const uint8_t* a = uniform_ptr(l.abase + kt * l.lda_kt);
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-    __builtin_amdgcn_global_load_lds(b + l.boff_src[h], (lds_void*)(st + TH::B_OFF + (2 * l.wave + h) * 1024), 16, 0, 0);
+    for (int j = 0; j < MB; ++j)
+      __builtin_amdgcn_global_load_lds(a + l.aoff_src[j], (lds_void*)(st + i * TH::A_STEP + (MB * l.wave + j) * 1024),
+                                       16, 0, 0);
+    __builtin_amdgcn_global_load_lds(uniform_ptr(l.sbase + kt * l.lds_kt) + l.soff_src,
+                                     (lds_void*)(st + 2 * TH::A_STEP + 256 * i), 4, 0, 0);
+  }
 }
 
 // `mul`: the wave's weight rows are not all past N.
-template <class C, int MB>
-__device__ __forceinline__ void mx_thin_kloop(f32x16_t (&acc)[MB][2], bool mul, int KT, uint8_t* smem,
-                                              const MxLane<C>& l) {
+template <int MB>
+__device__ __forceinline__ void mx_thin_kloop(f32x16_t (&acc)[MB][2], bool mul, uint8_t* smem, const MxLane& l) {
   using TH = MxThin<MB>;
-  for (int i = 0; i < TH::NS - 1; ++i)
-    if (i < KT) mx_thin_issue<C, MB>(smem, i, l);
-  for (int kt = 0; kt < KT; ++kt) {
-    // stage kt has landed for every wave, and every wave is done reading
-    // stage kt - 1, which takes step kt + NS - 1
-    wait_tiles_ahead<TH::PER, TH::NS - 2>(min(TH::NS - 2, KT - 1 - kt));
+  const int KT = l.KT, NPAIR = (KT + 1) >> 1;
+  mx_issue_scales(smem, 0, l);
+  mx_thin_issue_a<MB>(smem, 0, l);
+#pragma unroll
+  for (int i = 0; i < TH::NBP - 1; ++i)
+    if (i < NPAIR) mx_issue_b(smem + TH::B_OFF + i * MX_B_PAIR, i, l);
+  int bslot = 0;  // pair p's B stage
+  for (int p = 0; p < NPAIR; ++p) {
+    // pair p has landed for every wave (the B of pairs p + 1 .. p + NBP - 2
+    // may be in flight), and every wave is done reading pair p - 1
+    wait_tiles_ahead<MX_B_DMA, TH::NBP - 2>(min(TH::NBP - 2, NPAIR - 1 - p));
     wait_lgkm0();
     asm volatile("s_barrier" ::: "memory");
-    if (kt + TH::NS - 1 < KT) mx_thin_issue<C, MB>(smem, kt + TH::NS - 1, l);
-    if (!mul) continue;
-    const uint8_t* st = smem + (kt % TH::NS) * TH::STAGE;
-    MxB<2> b;
-    mx_read_b(b, st, l.boff, l.sb_row, l.G, kt);
-    MxA x[MB];
+    if (p % (MX_SC_STEPS / 2) == 0) mx_issue_scales(smem, p / (MX_SC_STEPS / 2) + 1, l);
+    if (p + 1 < NPAIR) mx_thin_issue_a<MB>(smem, p + 1, l);
+    if (p + TH::NBP - 1 < NPAIR)
+      mx_issue_b(smem + TH::B_OFF + (bslot == 0 ? TH::NBP - 1 : bslot - 1) * MX_B_PAIR, p + TH::NBP - 1, l);
+    if (mul) {
+      const uint8_t* sa = smem + (p & 1) * TH::A_PAIR;
+      const uint8_t* sb = smem + TH::B_OFF + bslot * MX_B_PAIR;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      mx_read_a(x[mb], st + mb * 4096, st + l.asoff + mb * 128, l.aoff0, l.aoff1, l.aoff2, l.aoff3);
+      for (int i = 0; i < 2; ++i) {
+        if (i == 1 && 2 * p + 1 >= KT) break;
+        MxB<2> b;
+        mx_read_b(b, sb, l, 2 * p + i);
+        MxA x[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) mx_mfma_row(acc[mb], x[mb], b);
+        for (int mb = 0; mb < MB; ++mb)
+          mx_read_a(x[mb], sa + i * TH::A_STEP + mb * 4096, sa + 2 * TH::A_STEP + 256 * i + l.asoff + mb * 128, l.aoff0,
+                    l.aoff1, l.aoff2, l.aoff3);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) mx_mfma_row(acc[mb], x[mb], b);
+      }
+    }
+    bslot = bslot + 1 == TH::NBP ? 0 : bslot + 1;
   }
   wait_vmcnt<0>();
   wait_lgkm0();
 }
 
+// The LDS offset of a lane's B operand in a pair (step parity 0) and of its
+// scale bytes, from its first weight row q of the tile.
+__device__ __forceinline__ void mx_lane_b(MxLane& l, const uint8_t* smem, int q, int kp) {
+  const int lh = l.lane >> 5;
+  l.boff = kp ? (uint32_t)((q >> 4) * 1024 + (q & 15) * 32 + ((lh ^ ((q >> 3) & 1)) * 16))
+              : (uint32_t)(q * 64 + ((lh ^ ((q >> 2) & 3)) * 16));
+  l.bpar = kp ? 512u : 32u;
+  l.sb_row = smem + MX_SC_OFF + q * MX_SC_ROW + ((l.bs_shift + min(q, l.bs_rows - 1) * l.G) & 3) + lh;
+}
+
 // The whole thin tile: `rows` (at most 32 MB) sorted rows from m0 against
 // weight rows n0 .. n0 + 255.  l holds what both forms share.
-template <int EPI, class C, int MB>
-__device__ __forceinline__ void mx_thin_tile(const GemmArgs& a, MxLane<C>& l, int e, int m0, int rows, int n0,
-                                             const uint8_t* sbs, uint8_t* smem) {
-  static_assert(C::W == 4 && C::BN == 256, "four waves of 64 weight rows");
+template <int EPI, int MB>
+__device__ __forceinline__ void mx_thin_tile(const GemmArgs& a, MxLane& l, int e, int m0, int rows, int n0,
+                                             uint8_t* smem) {
   const int l32 = l.lane & 31;
   const int lh = l.lane >> 5;
 #pragma unroll
@@ -2115,9 +2187,8 @@ __device__ __forceinline__ void mx_thin_tile(const GemmArgs& a, MxLane<C>& l, in
   l.aoff1 = (uint32_t)(l32 * 128 + (((2 + lh) ^ rsw) * 16));
   l.aoff2 = (uint32_t)(l32 * 128 + (((4 + lh) ^ rsw) * 16));
   l.aoff3 = (uint32_t)(l32 * 128 + (((6 + lh) ^ rsw) * 16));
-  l.asoff = (uint32_t)(MxThin<MB>::AS_OFF + l32 * 4 + lh);
-  l.boff = (uint32_t)(MxThin<MB>::B_OFF + bq[0] * 32 + ((lh ^ ((bq[0] >> 3) & 1)) * 16));
-  l.sb_row = sbs + bq[0] * l.G + lh;
+  l.asoff = (uint32_t)(l32 * 4 + lh);
+  mx_lane_b(l, smem, bq[0], a.kp);
   f32x16_t acc[MB][2];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -2125,24 +2196,13 @@ __device__ __forceinline__ void mx_thin_tile(const GemmArgs& a, MxLane<C>& l, in
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  mx_thin_kloop<C, MB>(acc, n0 + l.wave * 64 < a.N, a.K / MX_BK, smem, l);
+  mx_thin_kloop<MB>(acc, n0 + l.wave * 64 < a.N, smem, l);
   __syncthreads();
   epilogue_staged<EPI, MB, 2>(a, acc, bias, m0, 0, rows, n0 + l.wave * 64, smem + l.wave * epi_lds_bytes(MB, 2), l.lane);
 }
 
-template <int EPI, int MX_NS, bool SB16, int WM, int WN, int NB>
-__global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(GemmArgs a) {
-  static_assert(WM == 2, "two row blocks per wave (the split-step pipeline)");
-  using C = MxCfg<WN, NB>;
-  constexpr int W = C::W;
-  static_assert(MX_NS >= 2 && MX_NS <= 6, "pipeline depth");
-  static_assert(W == 4 || W == 8, "wave grid");
-  static_assert(C::B_DMA * W * 32 == C::BN, "B stage split over the waves");
-  static_assert(32 % C::AS_ROWS == 0, "whole scale slots per row block");
-  static_assert(MxThin<1>::NS * MxThin<1>::STAGE <= MX_NS * C::STAGE &&
-                    MxThin<2>::NS * MxThin<2>::STAGE <= MX_NS * C::STAGE,
-                "the thin tiles' stages fit below the B scales");
-  constexpr int BN = C::BN;
+template <int EPI>
+__global__ __launch_bounds__(64 * MX_W, 2) void moe_mx_kernel(GemmArgs a) {
   extern __shared__ __align__(1024) uint8_t smem[];
   const int L = xcd_tile_index(*a.num_tiles * a.n_tiles_n);
   if (L < 0) return;
@@ -2152,67 +2212,73 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   const int e = te.x;
   const int m0 = te.y;
   const int rows = min(MX_BM, a.offsets[e] + a.counts[e] - m0);
-  const int n0 = nt * BN;
+  const int n0 = nt * MX_BN;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN;   // rows 64*wm .. of the tile
-  const int wn = wave % WN;   // weight rows WCOLS*wn .. of the tile
+  const int wm = wave >> 1;   // rows 64*wm .. of the tile
+  const int wn = wave & 1;    // weight rows MX_WCOLS*wn .. of the tile
   const int G = a.K / 32;
-  const int KT = a.K / MX_BK;
   const int l32 = lane & 31;
   const int lh = lane >> 5;
-  uint8_t* sbs = smem + MX_NS * C::STAGE;  // [BN][G] B scales
-  preload_b_scales<SB16, BN, W>(a.Bs, e, a.N, n0, G, sbs, wave, lane);
 
-  // --- per-lane stage DMA sources (every lane always issues all of them, so
-  //     the per-wave vmcnt arithmetic is exact; rows or columns past the tile
-  //     are loaded from valid addresses and never stored) ------------------
-  MxLane<C> l;
+  // --- per-lane stage DMA sources (what a wave issues per step does not
+  //     depend on the data, so the per-wave vmcnt arithmetic is exact; rows
+  //     or columns past the tile are loaded from valid addresses and never
+  //     stored) ---------------------------------------------------------------
+  MxLane l;
   // A: the tile's 128 sorted rows of k-tile kt are one contiguous 16 KiB run
   // (rows past the valid ones belong to the next expert, or to the 128 spare
-  // rows at the end).  Instruction i = A_DMA*wave + j covers rows 8i .. 8i+7,
-  // 8 lanes per row; row r's chunk c lands in slot c ^ ((r >> 1) & 7).
+  // rows at the end).  Instruction i = 4*wave + j covers rows 8i .. 8i+7, 8
+  // lanes per row; row r's chunk c lands in slot c ^ ((r >> 1) & 7).
   l.abase = a.Aq + (int64_t)m0 * 128;
 #pragma unroll
-  for (int j = 0; j < C::A_DMA; ++j) {
-    const int r = 8 * (C::A_DMA * wave + j) + (lane >> 3);
+  for (int j = 0; j < MX_A_DMA; ++j) {
+    const int r = 8 * (MX_A_DMA * wave + j) + (lane >> 3);
     l.aoff_src[j] = (uint32_t)(r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) * 16));
   }
   // A scales: one dword (two scale bytes, two spare) per row; wave w's slot
-  // holds rows AS_ROWS*w .. +AS_ROWS (lanes past AS_ROWS repeat them)
+  // holds rows 32 w .. 32 w + 31 (lanes past 31 repeat them)
   l.sbase = a.As + (int64_t)m0 * 4;
-  l.soff_src = (uint32_t)((C::AS_ROWS * wave + lane % C::AS_ROWS) * 4);
-  // B: instruction i = B_DMA*wave + h covers rows 32i .. 32i+31, 2 lanes per
-  // row; row q's group g sits in half g ^ ((q >> 3) & 1) of its 32 bytes
+  l.soff_src = (uint32_t)((32 * wave + l32) * 4);
+  // B: instruction i = 4*wave + h covers rows 16i .. 16i+15, 4 lanes per row
+  // (checkpoint) or the two steps' 512-byte runs one after the other (k-pair)
   l.bbase = a.Bq + (int64_t)e * a.N * G * 16;
+  const int brow = a.kp ? (lane >> 1) & 15 : lane >> 2;
+  const int bgrp = a.kp ? 2 * (lane >> 5) + ((lane & 1) ^ (brow >> 3)) : (lane & 3) ^ ((lane >> 4) & 3);
 #pragma unroll
-  for (int h = 0; h < C::B_DMA; ++h) {
-    const int q = 32 * (C::B_DMA * wave + h) + (lane >> 1);
-    const int grp = (lane & 1) ^ ((q >> 3) & 1);
-    l.boff_src[h] = (uint32_t)bq_off(a.kp, n0 + q < a.N ? n0 + q : n0, grp, G);
+  for (int h = 0; h < MX_B_DMA; ++h) {
+    const int q = 16 * (MX_B_DMA * wave + h) + brow;
+    l.boff_src[h] = (uint32_t)bq_off(a.kp, n0 + q < a.N ? n0 + q : n0, bgrp, G);
   }
   l.lda_kt = a.ldq;
   l.lds_kt = a.ldas;
-  l.bkt = a.kp ? 512 : 32;  // bytes per k-tile (two groups) along a row
+  l.bpair = a.kp ? 1024 : 64;  // bytes per pair of k-tiles (four groups) along a row
+  l.bback = bgrp < 2 ? 0 : (a.kp ? 512 : 32);
+  const int64_t s0 = ((int64_t)e * a.N + n0) * G;
+  l.bs = a.Bs + (s0 & ~(int64_t)3);
+  l.bs_shift = (int)(s0 & 3);
+  l.bs_rows = min(MX_BN, a.N - n0);
+  l.bs_last = (int)min((((int64_t)a.E * a.N * G - 1) & ~(int64_t)3) - (s0 & ~(int64_t)3), (int64_t)1 << 30);
+  l.KT = a.K / MX_BK;
   l.wave = wave;
   l.lane = lane;
   l.G = G;
 
   if (rows <= 64) {
     if (rows <= 32)
-      mx_thin_tile<EPI, C, 1>(a, l, e, m0, rows, n0, sbs, smem);
+      mx_thin_tile<EPI, 1>(a, l, e, m0, rows, n0, smem);
     else
-      mx_thin_tile<EPI, C, 2>(a, l, e, m0, rows, n0, sbs, smem);
+      mx_thin_tile<EPI, 2>(a, l, e, m0, rows, n0, smem);
     return;
   }
 
   // this lane's B rows (one per 32-column block) and their bias
-  int bq[NB];
-  float bias[NB];
+  int bq[MX_NB];
+  float bias[MX_NB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    bq[nb] = wn * C::WCOLS + nb * 32 + l32;
+  for (int nb = 0; nb < MX_NB; ++nb) {
+    bq[nb] = wn * MX_WCOLS + nb * 32 + l32;
     const bool ok = n0 + bq[nb] < a.N;
     bias[nb] = ok ? bias_at(a.bias, a.bias_dtype, (int64_t)e * a.N + n0 + bq[nb]) : 0.f;
   }
@@ -2225,18 +2291,15 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   l.aoff1 = abase + (uint32_t)(((2 + lh) ^ rsw) * 16);
   l.aoff2 = abase + (uint32_t)(((4 + lh) ^ rsw) * 16);
   l.aoff3 = abase + (uint32_t)(((6 + lh) ^ rsw) * 16);
-  // the row's scale byte lh in its wave slot (row block 1: + AS_BLOCK)
-  const int srow = 64 * wm + l32;
-  l.asoff = (uint32_t)(MX_A_BYTES + (srow / C::AS_ROWS) * 256 + (srow % C::AS_ROWS) * 4 + lh);
-  // B: half lh ^ bsw of row bq (bsw = bit 3 of the row, the same for every nb)
-  l.boff = (uint32_t)(C::B_OFF + bq[0] * 32 + ((lh ^ ((bq[0] >> 3) & 1)) * 16));
-  l.sb_row = sbs + bq[0] * G + lh;  // + nb*32*G + 2kt
+  // the row's scale byte lh in its slot (row block 1: the next slot)
+  l.asoff = (uint32_t)(MX_A_BYTES + 2 * wm * 256 + l32 * 4 + lh);
+  mx_lane_b(l, smem, bq[0], a.kp);
 
-  f32x16_t acc[2][NB];
+  f32x16_t acc[2][MX_NB];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+    for (int j = 0; j < MX_NB; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
@@ -2244,25 +2307,25 @@ __global__ __launch_bounds__(64 * WM * WN, BSA_MX_WG_PER_CU) void moe_mx_kernel(
   // wave's row blocks holding rows of the tile, uniform across the wave; the
   // loop's barrier count does not depend on it).  Nor is anything of a wave
   // whose weight rows all lie past N (in the last column tile: half of it at
-  // gate_up's N = 5760, and at down's N = 2880).
-  const int nmb = n0 + wn * C::WCOLS < a.N ? min(2, max(0, (rows - 64 * wm + 31) / 32)) : 0;
-  // The wave's share of the A stage is left out when it lies past the tile's
-  // rows: a tile of one 32-row block then streams 12 KiB a step, not 24.
-  const bool al = 8 * C::A_DMA * wave < rows;
+  // gate_up's N = 5760, and at down's N = 2880).  The wave's share of the A
+  // stage (rows 32 wave ..) is left out when it lies past the tile's rows.
+  const int nmb = n0 + wn * MX_WCOLS < a.N ? min(2, max(0, (rows - 64 * wm + 31) / 32)) : 0;
+  const bool al = 32 * wave < rows;
   if (nmb == 2)
-    mx_kloop<C, MX_NS, 2, true>(acc, KT, smem, l);
+    mx_kloop<2, true>(acc, smem, l);
   else if (nmb == 1 && al)
-    mx_kloop<C, MX_NS, 1, true>(acc, KT, smem, l);
+    mx_kloop<1, true>(acc, smem, l);
   else if (nmb == 1)
-    mx_kloop<C, MX_NS, 1, false>(acc, KT, smem, l);
+    mx_kloop<1, false>(acc, smem, l);
   else if (al)
-    mx_kloop<C, MX_NS, 0, true>(acc, KT, smem, l);
+    mx_kloop<0, true>(acc, smem, l);
   else
-    mx_kloop<C, MX_NS, 0, false>(acc, KT, smem, l);
+    mx_kloop<0, false>(acc, smem, l);
 
   // epilogue through LDS: the stage buffers are free once every wave is done
   __syncthreads();
-  epilogue_staged<EPI, 2, NB>(a, acc, bias, m0, 64 * wm, rows, n0 + wn * C::WCOLS, smem + wave * C::EPI_LDS, lane);
+  epilogue_staged<EPI, 2, MX_NB>(a, acc, bias, m0, 64 * wm, rows, n0 + wn * MX_WCOLS,
+                                 smem + wave * epi_lds_bytes(2, MX_NB), lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2755,7 +2818,7 @@ static int allow_big_lds(const void* fn, int kind, int epi, int bytes = 160 * 10
     return BSA_EHIP;
   }
   // kinds: 1-3 packed-weight backward kernel, 4-5 tiled kernel, 6-7 persistent
-  // decode kernel, 8-15 MX kernel configurations
+  // decode kernel, 8 MX kernel
   static bool allowed[64][16][8];
   if (!allowed[dev][kind][epi]) {
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -2767,53 +2830,9 @@ static int allow_big_lds(const void* fn, int kind, int epi, int bytes = 160 * 10
   return BSA_OK;
 }
 
-template <int EPI, int NS, int WM, int WN, int NB>
-static int launch_mx_cfg(const GemmArgs& a, int64_t P, size_t smem, hipStream_t st) {
-  using C = MxCfg<WN, NB>;
-  const int64_t max_tiles = (P + MX_BM - 1) / MX_BM + a.E;
-  GemmArgs b = a;
-  b.n_tiles_n = (a.N + C::BN - 1) / C::BN;
-  const int64_t grid = align_up(max_tiles * b.n_tiles_n, 8);
-  if (grid > INT32_MAX) {
-    set_error("MX GEMM: grid too large");
-    return BSA_EINVAL;
-  }
-  const bool sb16 = reinterpret_cast<uintptr_t>(a.Bs) % 16 == 0;
-  const void* fn = sb16 ? reinterpret_cast<const void*>(moe_mx_kernel<EPI, NS, true, WM, WN, NB>)
-                        : reinterpret_cast<const void*>(moe_mx_kernel<EPI, NS, false, WM, WN, NB>);
-  int rc = allow_big_lds(fn, 8 + (sb16 ? 1 : 0), EPI);
-  if (rc) return rc;
-  if (sb16)
-    hipLaunchKernelGGL((moe_mx_kernel<EPI, NS, true, WM, WN, NB>), dim3((unsigned)grid), dim3(64 * C::W), smem,
-                       st, b);
-  else
-    hipLaunchKernelGGL((moe_mx_kernel<EPI, NS, false, WM, WN, NB>), dim3((unsigned)grid), dim3(64 * C::W),
-                       smem, st, b);
-  BSA_LAUNCH_CHECK("MX grouped GEMM launch");
-  return BSA_OK;
-}
-
 // Block-scaled MX grouped GEMM (K % 64 == 0; 16-byte aligned blocks, 4-byte
 // aligned weight scales; a.Aq / a.As the k-tile-major split of the sorted
 // activation rows, with 128 spare rows after the last).
-// Pipeline depth BSA_MX_NS, a 2 x BSA_MX_WN wave grid with BSA_MX_NB
-// 32-column blocks per wave (a build-time choice; the defaults measured
-// fastest at the gpt-oss-120b prefill shapes: a third stage does not fit two
-// workgroups per CU, and 8-wave grids at one workgroup per CU ran 7-10%
-// slower).  BSA_MX_WM stays 2: the split-step pipeline multiplies two row
-// blocks per wave.
-#ifndef BSA_MX_NS
-#define BSA_MX_NS 2
-#endif
-#ifndef BSA_MX_WM
-#define BSA_MX_WM 2
-#endif
-#ifndef BSA_MX_WN
-#define BSA_MX_WN 2
-#endif
-#ifndef BSA_MX_NB
-#define BSA_MX_NB 4
-#endif
 template <int EPI>
 static int launch_gemm_mx(const GemmArgs& a, int64_t P, hipStream_t st) {
   if (a.K % MX_BK != 0 || reinterpret_cast<uintptr_t>(a.Bq) % 16 != 0 ||
@@ -2823,15 +2842,21 @@ static int launch_gemm_mx(const GemmArgs& a, int64_t P, hipStream_t st) {
               a.K);
     return BSA_EINVAL;
   }
-  using C = MxCfg<BSA_MX_WN, BSA_MX_NB>;
-  // the epilogue stages each wave's results in the (then idle) stages and
-  // B-scale buffer
-  const size_t smem = std::max(mx_smem_bytes<C>(BSA_MX_NS, a.K), (size_t)C::W * C::EPI_LDS);
-  if (smem > 160 * 1024) {
-    set_error("MX GEMM: K=%d needs %zu bytes of LDS", a.K, smem);
+  // the epilogue stages each wave's results in the (then idle) stages
+  static_assert(MX_W * epi_lds_bytes(2, MX_NB) <= MX_SMEM, "epilogue staging");
+  const int64_t max_tiles = (P + MX_BM - 1) / MX_BM + a.E;
+  GemmArgs b = a;
+  b.n_tiles_n = (a.N + MX_BN - 1) / MX_BN;
+  const int64_t grid = align_up(max_tiles * b.n_tiles_n, 8);
+  if (grid > INT32_MAX) {
+    set_error("MX GEMM: grid too large");
     return BSA_EINVAL;
   }
-  return launch_mx_cfg<EPI, BSA_MX_NS, BSA_MX_WM, BSA_MX_WN, BSA_MX_NB>(a, P, smem, st);
+  int rc = allow_big_lds(reinterpret_cast<const void*>(moe_mx_kernel<EPI>), 8, EPI, MX_SMEM);
+  if (rc) return rc;
+  hipLaunchKernelGGL((moe_mx_kernel<EPI>), dim3((unsigned)grid), dim3(64 * MX_W), MX_SMEM, st, b);
+  BSA_LAUNCH_CHECK("MX grouped GEMM launch");
+  return BSA_OK;
 }
 
 // Compute units of the current device (cached per device).
@@ -2879,10 +2904,11 @@ static int run_dispatch(const int64_t* idx, int64_t P, int E, const Workspace& w
 // Row groups (16-row blocks sharing one read of the weights) of the
 // persistent kernel: two once experts commonly hold more than 16 rows.  120b
 // layer, one against two (unevenly hit experts): 64 tokens 199 / 218 us, 128
-// 245 / 252, 256 338 / 325, 512 514 / 420.  (Four waves' operands of 32 rows do
+// 245 / 252, 256 338 / 325, 512 514 / 420; on k-pair blocks 200 tokens 297 /
+// 310.  (Four waves' operands of 32 rows do
 // not fit a wave's registers, so two groups take 512 threads and the CU's
 // whole ring, which the smaller batches, with fewer rows to share, pay for.)
-static int ps_row_groups(int64_t P, int64_t E) { return P > 6 * E ? 2 : 1; }
+static int ps_row_groups(int64_t P, int64_t E) { return P > 8 * E ? 2 : 1; }
 
 template <int EPI, int RG>
 static int launch_persist(const GemmArgs& a, int cus, hipStream_t st) {
@@ -3030,14 +3056,38 @@ struct MoeShape {
 // other side of the SwiGLU clamps from float32 (measured at the gpt-oss-120b
 // prefill shape: 246 against 26 of 189M), and each such flip moves a token's
 // input gradient by the size of its largest entries.
-static int resolve_path(int path, const MoeShape& m, const void* gu_b, const void* gu_s, const void* dn_b,
-                        const void* dn_s, bool saving) {
+//
+// Where both projections run the persistent streaming kernel, whose 32-row
+// passes read the weights at close to the HBM rate, it keeps the batch up to 32
+// rows per expert on average (120b layer, stream / MX: 700 tokens 493 / 563 us,
+// 1000 575 / 592, 1400 714 / 613; 32 experts: 256 tokens 174 / 187, 400 tokens
+// 230 / 219); elsewhere the MX kernels start at 16.
+static int resolve_path(int path, const MoeShape& m, const void* gu_b, const void* gu_s, const void* gu_bias,
+                        const void* dn_b, const void* dn_s, const void* dn_bias, bool saving) {
   if (path != PATH_AUTO || saving) return path;
   const bool a16 = reinterpret_cast<uintptr_t>(gu_b) % 16 == 0 && reinterpret_cast<uintptr_t>(dn_b) % 16 == 0;
   const bool s4 = reinterpret_cast<uintptr_t>(gu_s) % 4 == 0 && reinterpret_cast<uintptr_t>(dn_s) % 4 == 0;
   const int64_t P = m.T * m.k;
-  if (P > 16 * m.E && m.H % MX_BK == 0 && m.I % MX_BK == 0 && a16 && s4) return PATH_MX;
-  return PATH_AUTO;
+  if (P <= 16 * m.E || m.H % MX_BK != 0 || m.I % MX_BK != 0 || !a16 || !s4) return PATH_AUTO;
+  if (P <= 32 * m.E) {
+    GemmArgs g{};
+    g.E = (int)m.E;
+    g.N = (int)(2 * m.I);
+    g.K = (int)m.H;
+    g.lda = m.H;
+    g.Bq = static_cast<const uint8_t*>(gu_b);
+    g.Bs = static_cast<const uint8_t*>(gu_s);
+    g.bias = gu_bias;
+    GemmArgs d = g;
+    d.N = (int)m.H;
+    d.K = (int)m.I;
+    d.lda = m.I;
+    d.Bq = static_cast<const uint8_t*>(dn_b);
+    d.Bs = static_cast<const uint8_t*>(dn_s);
+    d.bias = dn_bias;
+    if (persist_ok(g, P) && persist_ok(d, P)) return PATH_STREAM;
+  }
+  return PATH_MX;
 }
 
 static int check_shape(const MoeShape& m, const char* what) {
@@ -3335,7 +3385,8 @@ static int experts_fwd(
       (rc = check_layout(blocks_layout, down_blocks, H, I, "experts fwd (down)")))
     return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  path = resolve_path(path, m, gate_up_blocks, gate_up_scales, down_blocks, down_scales, save_swiglu_grad != nullptr);
+  path = resolve_path(path, m, gate_up_blocks, gate_up_scales, gate_up_bias, down_blocks, down_scales, down_bias,
+                      save_swiglu_grad != nullptr);
   if (noalloc) {
     workspace_bytes = carve(nullptr, T, H, I, E, k).bytes;
     BSA_REQUIRE(workspace_bytes <= NOALLOC_SCRATCH_BYTES,

@@ -393,11 +393,16 @@ int launch_dispatch(const int64_t* idx, int P, int E, int BM, int* counts, int* 
   return BSA_OK;
 }
 
+// Tokens from which one workgroup per token, all its loads in flight, is at
+// least as fast as one per 1024-column slice (120b layer: 64 tokens 7.0 / 7.3
+// us, 512 7.1 / 11.9, 1000 10.5 / 22.3).
+constexpr int COMBINE4_T = 256;
+
 int launch_combine(const float* Y, const int64_t* idx, const void* w, int w_dtype,
                    const int* pair_pos, int T, int k, int H, void* out, int out_dtype,
                    hipStream_t st) {
   if (T == 0) return BSA_OK;
-  if (T >= 1024 && k <= 4 && H % 4 == 0 && H <= 4096 && reinterpret_cast<uintptr_t>(Y) % 16 == 0 &&
+  if (T >= COMBINE4_T && k <= 4 && H % 4 == 0 && H <= 4096 && reinterpret_cast<uintptr_t>(Y) % 16 == 0 &&
       (out_dtype != DT_BF16 || reinterpret_cast<uintptr_t>(out) % 8 == 0)) {
     const int it = (H + 1023) / 1024;
     auto fn = it == 1 ? moe_combine4_kernel<1>

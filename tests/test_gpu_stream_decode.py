@@ -151,7 +151,7 @@ def test_persistent_two_row_groups_edges(device, rows):
     idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(
         T, generator=torch.Generator().manual_seed(1))].reshape(T, k).to(device)
     w = torch.full((T, k), 0.5, dtype=torch.bfloat16, device=device)
-    assert T * k > 6 * E
+    assert T * k > 8 * E
     announce(f"persistent kernel, two row groups, counts {counts}")
     persist, parts = _both_kernels(t, idx, w)
     _agree(persist, parts, f"counts {counts}")
