@@ -74,6 +74,32 @@ def test_backward_vs_oracle_autograd(device, case):
     assert_grad_close(gw, rw, f"d routing weights {case}")
 
 
+@pytest.mark.parametrize("layout", ["checkpoint", "kpair"])
+@pytest.mark.parametrize("H,I", [(640, 576), (576, 544), (64, 32)], ids=["H640I576", "H576I544", "H64I32"])
+def test_backward_few_rows_per_expert(device, H, I, layout):
+    """The streaming backward kernel at the edges of its 16-row groups and 64-row passes, beside experts
+    without rows, with column tiles of 512 columns and a rest, and with fewer k-steps than waves."""
+    if layout == "kpair" and I % 64:
+        pytest.skip("the k-pair layout needs an even number of 32-element groups")
+    counts = [1, 16, 17, 0, 32, 33, 64, 65]
+    E, T = 32, sum(counts)  # 8 rows per expert at most: the streaming kernel
+    assert T <= 8 * E
+    t = synthetic.moe_layer(synthetic.MoEShape(E, 1, H, I, T), seed=H, scale_lo=116, scale_hi=120, device=device)
+    gen = torch.Generator().manual_seed(I)
+    idx = torch.repeat_interleave(torch.arange(len(counts)) * 4 + 3, torch.tensor(counts))[torch.randperm(T, generator=gen)]
+    idx = idx[:, None].to(device)
+    w = (torch.rand(T, 1, generator=gen) + 0.5).to(device)
+    g = torch.randn(T, H, generator=gen).to(torch.bfloat16).to(device)
+    announce(f"moe backward, few rows per expert, {H} x {I}, {layout}")
+    _, rh, rw = _oracle_grads(t, idx, w, g)
+    if layout == "kpair":
+        for name in ("gate_up_proj_blocks", "down_proj_blocks"):
+            t[name] = kernels.to_kpair(t[name])
+    _, gh, gw = _gpu_grads(t, idx, w, g)
+    assert_grad_close(gh, rh, "d hidden")
+    assert_grad_close(gw, rw, "d routing weights")
+
+
 def test_backward_through_module_like_recompute(device):
     """functional_call + autograd.grad on [hidden, weights], as _autograd.py:127-175 does."""
     from torch.func import functional_call
