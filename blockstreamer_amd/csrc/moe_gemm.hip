@@ -2893,7 +2893,10 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
   };
   Step t[D];
 #pragma unroll
-  for (int d = 0; d < D - 1; ++d) load(t[d], d);
+  for (int d = 0; d < D - 1; ++d) {
+    load(t[d], d);
+    __builtin_amdgcn_sched_barrier(0);  // in the loop's order, which its first wait counts on
+  }
   for (int s = 0; s < n; s += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -3029,9 +3032,10 @@ static int launch_gemm_packed_rows(const GemmArgs& a, int64_t P, hipStream_t st)
   // 120b layer, this kernel against the 128-row one: 8 rows per expert (256
   // tokens) 787 / 866 us, 16 (512) 1069 / 1157, 24 (760) 1624 / 1276; with 32
   // experts, whose tiles leave a quarter of the CUs idle, 8 (64) 250 / 273, 16
-  // (128) 382 / 345.
+  // (128) 382 / 345.  One expert (mxfp4_matmul's transposed product, 5760 x
+  // 2880): 1 to 8 rows 44 / 100 us.
   const bool b32 = (int64_t)a.K * a.N / 2 <= INT32_MAX && (int64_t)BS_ROWS * a.lda * 2 <= INT32_MAX;
-  if (q16 && b32 && P <= ((int64_t)a.E * b.n_tiles_n >= 512 ? 16 : 8) * (int64_t)a.E) {
+  if (q16 && b32 && P <= (a.E == 1 || (int64_t)a.E * b.n_tiles_n >= 512 ? 16 : 8) * (int64_t)a.E) {
     void (*fn)(GemmArgs) = a.kp ? moe_bwd_stream_kernel<EPI, true> : moe_bwd_stream_kernel<EPI, false>;
     int rc = allow_big_lds(reinterpret_cast<const void*>(fn), a.kp ? 10 : 9, EPI, BS_SMEM);
     if (rc) return rc;
@@ -3147,10 +3151,11 @@ static int run_dispatch(const int64_t* idx, int64_t P, int E, const Workspace& w
 // persistent kernel: two once experts commonly hold more than 16 rows.  120b
 // layer, one against two (unevenly hit experts): 64 tokens 199 / 218 us, 128
 // 245 / 252, 256 338 / 325, 512 514 / 420; on k-pair blocks 200 tokens 297 /
-// 310.  (Four waves' operands of 32 rows do
-// not fit a wave's registers, so two groups take 512 threads and the CU's
+// 310.  With few experts the line lies later: 32 experts, 66 tokens 105 / 120
+// us, 72 116 / 120, 80 121 / 119, 128 144 / 132.  (Four waves' operands of 32
+// rows do not fit a wave's registers, so two groups take 512 threads and the CU's
 // whole ring, which the smaller batches, with fewer rows to share, pay for.)
-static int ps_row_groups(int64_t P, int64_t E) { return P > 8 * E ? 2 : 1; }
+static int ps_row_groups(int64_t P, int64_t E) { return P > (E >= 64 ? 8 : 10) * E ? 2 : 1; }
 
 template <int EPI, int RG>
 static int launch_persist(const GemmArgs& a, int cus, hipStream_t st) {
