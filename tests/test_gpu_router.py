@@ -90,6 +90,36 @@ def test_router_bf16_module(device, T, E, k):
     assert torch.equal(idx.cpu()[clear], ri[clear])
 
 
+@pytest.mark.parametrize("T,H,E,k", [(4128, 2880, 128, 4), (4097, 160, 32, 4), (4111, 32, 5, 5), (4130, 96, 33, 3),
+                                     (4096, 288, 64, 8), (4099, 640, 100, 16)])
+def test_router_one_launch(device, T, H, E, k):
+    """The one-launch router of long prompts: token and expert remainders, fewer k-steps than a wave's
+    loads in flight, ties, infinities and NaN.  More than 128 experts take the separate kernels, whose
+    sums run in the same order: both must give the same bits."""
+    gen = torch.Generator().manual_seed(T + E)
+    h = torch.randn(T, H, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(160, H, generator=gen) * 0.05).to(torch.bfloat16)
+    b = (torch.randn(160, generator=gen) * 0.5).to(torch.bfloat16)
+    b[1] = b[0]
+    h[0] = 0.0                     # logits are the biases: a tie
+    h[1] = float("nan")
+    h[T - 1, 0] = float("inf")
+    h, w, b = h.to(device), w.to(device), b.to(device)
+    announce(f"one-launch router T={T} H={H} E={E} k={k}")
+    logits, scores, idx = kernels.router_forward(h, w[:E].contiguous(), b[:E].contiguous(), k)
+    want = kernels.router_forward(h, w, b, k)[0][:, :E].contiguous()
+    assert torch.equal(logits.isnan(), want.isnan())
+    assert torch.equal(logits.nan_to_num(nan=0.0).view(torch.int16), want.nan_to_num(nan=0.0).view(torch.int16))
+    want_scores, want_idx = kernels.router_topk(logits, k)
+    assert torch.equal(idx, want_idx)
+    assert torch.equal(scores.view(torch.int16), want_scores.view(torch.int16))
+    ok = torch.arange(2, T - 1)
+    ref = h.cpu()[ok].double() @ w.cpu()[:E].double().t() + b.cpu()[:E].double()
+    # one bf16 rounding, and float32 sums of H products
+    bound = ref.abs() * 2 ** -8 + 2 ** -24 * H * (h.cpu()[ok].double().abs() @ w.cpu()[:E].double().abs().t())
+    assert ((logits.cpu()[ok].double() - ref).abs() <= bound + 1e-6).all()
+
+
 def test_router_backward_vs_transformers(device):
     gpt_oss = pytest.importorskip("transformers.models.gpt_oss.modeling_gpt_oss")
     from transformers.models.gpt_oss.configuration_gpt_oss import GptOssConfig
