@@ -770,13 +770,6 @@ __device__ __forceinline__ void at_dkv_unit(const uint8_t* T, bool full, uint32_
     sc = at_mfma(*reinterpret_cast<const u32x4_t*>(T + aoff[s]), kf[s], sc);
     dp = at_mfma(*reinterpret_cast<const u32x4_t*>(DO + aoff[s]), vf[s], dp);
   }
-  if (!full) {  // hidden scores to -inf: their P and dS are 0
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const uint32_t k = at_vis_mask(vis, v);
-      sc[v] = __uint_as_float((k & __float_as_uint(sc[v])) | (~k & 0xFF800000u));
-    }
-  }
   u32x4_t pf[2], sf[2];
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
@@ -796,6 +789,19 @@ __device__ __forceinline__ void at_dkv_unit(const uint8_t* T, bool full, uint32_
       pf[half][i] = at_pack2(p[2 * i], p[2 * i + 1]);
       sf[half][i] = at_pack2(ds[2 * i], ds[2 * i + 1]);
     }
+  }
+  // Hidden P and dS to 0, as packed pairs: whatever the scaling's sign and
+  // whatever (L, D) a row has, nothing of it reaches a key it does not see.
+  if (!full) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t lo = at_vis_mask(vis, 8 * half + 2 * i), hi = at_vis_mask(vis, 8 * half + 2 * i + 1);
+        const uint32_t k = (lo & 0xFFFFu) | (hi & 0xFFFF0000u);
+        pf[half][i] &= k;
+        sf[half][i] &= k;
+      }
   }
 #pragma unroll
   for (int s = 0; s < 2; ++s)

@@ -402,3 +402,43 @@ def test_attention_far_strides(device):
     assert torch.equal(out, want_out)
     for a, b in zip(got[:3], want[:3]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("scaling", [-0.125, 0.0, 0.125])
+@pytest.mark.parametrize("Tq,Hq,Hkv", [(40, 4, 4), (33, 24, 8), (101, 8, 1)])
+def test_backward_hidden_rows_whatever_the_scaling(device, scaling, Tq, Hq, Hkv):
+    """No mask, but units of 32 rows that end early (Tq * G no multiple of 32): the rows past the end add nothing
+    to dk and dv, also where the scaling is not positive."""
+    Tk = 128
+    announce(f"attention bwd scaling={scaling} Tq={Tq} Hq={Hq} Hkv={Hkv}")
+    assert Tq * (Hq // Hkv) % 32
+    q, k, v, s = _inputs(1, Hq, Hkv, Tq, Tk, device, seed=Tq + Hq)
+    dout = torch.randn(1, Tq, Hq, 64, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(device)
+    out, lse = A.attention_forward(q, k, v, s, scaling, return_lse=True)
+    got = A.attention_backward(dout, q, k, v, s, out, lse, scaling)
+    qr, kr, vr = (t.detach().cpu().double().requires_grad_(True) for t in (q, k, v))
+    ref = oracle.attention_ref(qr, kr, vr, s.cpu().double(), scaling)
+    ref.backward(dout.double().cpu())
+    assert _rel_l2(out, ref) <= BWD_REL_L2
+    for name, a, want in zip(("dq", "dk", "dv"), got, (qr.grad, kr.grad, vr.grad)):
+        assert torch.isfinite(a).all(), name
+        assert _rel_l2(a, want) <= BWD_REL_L2, name
+
+
+@pytest.mark.parametrize("window", [0, 20])
+def test_backward_nan_row_stays_with_the_keys_it_sees(device, window):
+    """A row of NaN (its query, so its log-denominator) leaves dv of every key it does not see as it was."""
+    announce(f"attention bwd NaN row window={window}")
+    T, t0, Hq, Hkv = 160, 70, 8, 1
+    q, k, v, s = _inputs(1, Hq, Hkv, T, T, device, seed=12)
+    dout = torch.randn(1, T, Hq, 64, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(device)
+    grads = []
+    for value in (0.0, float("nan")):
+        q2 = q.clone()
+        q2[:, :, t0] = value
+        out, lse = A.attention_forward(q2, k, v, s, 0.125, True, window, return_lse=True)
+        grads.append(A.attention_backward(dout, q2, k, v, s, out, lse, 0.125, True, window)[2][0, 0])
+    hidden = torch.ones(T, dtype=torch.bool)
+    hidden[t0 - window + 1 if window else 0:t0 + 1] = False
+    assert torch.equal(grads[1][hidden.to(device)], grads[0][hidden.to(device)])
+    assert torch.isnan(grads[1][t0]).all()
