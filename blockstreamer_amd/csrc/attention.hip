@@ -1033,6 +1033,10 @@ static int at_check_common(const char* what, int64_t B, int64_t Tq, int64_t Tk, 
   return BSA_OK;
 }
 
+// A window that reaches past every key hides none: 0 (no window), which also
+// keeps key + window within 32 bits.
+static int at_window(int64_t window, int64_t Tk) { return window >= Tk ? 0 : (int)window; }
+
 static int at_check_strides(const char* what, const int64_t* const* st, int n) {
   for (int j = 0; j < n; ++j)
     for (int i = 0; i < 3; ++i)
@@ -1106,7 +1110,7 @@ static int at_fwd_args(AttnArgs& a, const void* q, const int64_t* q_strides, con
   a.Hkv = (int)Hkv;
   a.G = (int)(Hq / Hkv);
   a.causal = causal ? 1 : 0;
-  a.window = (int)window;
+  a.window = at_window(window, Tk);
   a.scale2 = scaling * 1.4426950408889634f;
   a.nsplit = 1;
   return BSA_OK;
@@ -1256,7 +1260,7 @@ static int at_bwd(const void* grad_out, const int64_t* grad_strides, const void*
   a.Hkv = (int)Hkv;
   a.G = (int)(Hq / Hkv);
   a.causal = causal ? 1 : 0;
-  a.window = (int)window;
+  a.window = at_window(window, Tk);
   a.scale2 = scaling * 1.4426950408889634f;
   a.scaling = scaling;
   hipStream_t s = static_cast<hipStream_t>(stream);

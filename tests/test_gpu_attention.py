@@ -442,3 +442,22 @@ def test_backward_nan_row_stays_with_the_keys_it_sees(device, window):
     hidden[t0 - window + 1 if window else 0:t0 + 1] = False
     assert torch.equal(grads[1][hidden.to(device)], grads[0][hidden.to(device)])
     assert torch.isnan(grads[1][t0]).all()
+
+
+@pytest.mark.parametrize("window", [299, 300, 301, 2 ** 31 - 129, 2 ** 31 - 2])
+def test_window_past_every_key_is_no_window(device, window):
+    """A window of the sequence's length or more, up to the largest accepted, gives the causal results and gradients."""
+    announce(f"attention window={window}")
+    T, Hq, Hkv = 300, 16, 2
+    q, k, v, s = _inputs(1, Hq, Hkv, T, T, device, seed=31)
+    dout = torch.randn(1, T, Hq, 64, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(device)
+    res = []
+    for w in (0, window):
+        out, lse = A.attention_forward(q, k, v, s, 0.125, True, w, return_lse=True)
+        res.append((out, *A.attention_backward(dout, q, k, v, s, out, lse, 0.125, True, w)[:3]))
+    for name, a, want in zip(("out", "dq", "dk", "dv"), res[1], res[0]):
+        if window >= T and name in ("out", "dq"):
+            assert torch.equal(a, want), name
+        # the row splits of dk and dv may differ: the same float32 terms in another order and
+        # a flipped bf16 rounding here and there; a window of T - 1 hides one key from one query
+        assert _rel_l2(a, want) <= (2.0 ** -9 if window >= T else 2.0 ** -5), name
