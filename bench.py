@@ -259,12 +259,11 @@ def fp32_reference(x, idx, w, args, alpha=1.702, limit=7.0):
 def _resolved_kernel(path: str, T: int, wl: Workload) -> str:
     """The expert GEMM kernels an inference forward runs for ``path`` (the
     library's rule: automatic selection takes the MX kernels above 16 rows
-    per expert when H and I are multiples of 64, above 32 where the persistent
-    streaming kernel can run (H = I = 2880) -- the bench's weights are aligned;
-    a forward saving for the backward keeps the bf16 kernels)."""
+    per expert when H and I are multiples of 64 -- the bench's weights are
+    aligned; a forward saving for the backward keeps the bf16 kernels)."""
     if path != "auto":
         return path
-    if T * wl.k <= (32 if wl.H == wl.I == 2880 else 16) * wl.E:
+    if T * wl.k <= 16 * wl.E:
         return "stream"
     return "mx" if wl.H % 64 == 0 and wl.I % 64 == 0 else "tiled"
 

@@ -3304,37 +3304,20 @@ struct MoeShape {
 // prefill shape: 246 against 26 of 189M), and each such flip moves a token's
 // input gradient by the size of its largest entries.
 //
-// Where both projections run the persistent streaming kernel, whose 32-row
-// passes read the weights at close to the HBM rate, it keeps the batch up to 32
-// rows per expert on average (120b layer, stream / MX: 700 tokens 493 / 563 us,
-// 1000 575 / 592, 1400 714 / 613; 32 experts: 256 tokens 174 / 187, 400 tokens
-// 230 / 219); elsewhere the MX kernels start at 16.
-static int resolve_path(int path, const MoeShape& m, const void* gu_b, const void* gu_s, const void* gu_bias,
-                        const void* dn_b, const void* dn_s, const void* dn_bias, bool saving) {
+// The line is 16 rows per expert on average, whatever the widths.  The host
+// knows the average only: the streaming kernel reads an expert's weights once
+// per 32 rows, this path once per 128, so above the line a batch concentrated
+// on few experts pays for streaming (120b layer, stream / MX: 520 tokens spread
+// over the experts 428 / 506 us, on 16 of them 251 / 203, on 4 235 / 147; 1000
+// tokens 584 / 572, 417 / 253, 331 / 225).
+static int resolve_path(int path, const MoeShape& m, const void* gu_b, const void* gu_s, const void* dn_b,
+                        const void* dn_s, bool saving) {
   if (path != PATH_AUTO || saving) return path;
   const bool a16 = reinterpret_cast<uintptr_t>(gu_b) % 16 == 0 && reinterpret_cast<uintptr_t>(dn_b) % 16 == 0;
   const bool s4 = reinterpret_cast<uintptr_t>(gu_s) % 4 == 0 && reinterpret_cast<uintptr_t>(dn_s) % 4 == 0;
   const int64_t P = m.T * m.k;
-  if (P <= 16 * m.E || m.H % MX_BK != 0 || m.I % MX_BK != 0 || !a16 || !s4) return PATH_AUTO;
-  if (P <= 32 * m.E) {
-    GemmArgs g{};
-    g.E = (int)m.E;
-    g.N = (int)(2 * m.I);
-    g.K = (int)m.H;
-    g.lda = m.H;
-    g.Bq = static_cast<const uint8_t*>(gu_b);
-    g.Bs = static_cast<const uint8_t*>(gu_s);
-    g.bias = gu_bias;
-    GemmArgs d = g;
-    d.N = (int)m.H;
-    d.K = (int)m.I;
-    d.lda = m.I;
-    d.Bq = static_cast<const uint8_t*>(dn_b);
-    d.Bs = static_cast<const uint8_t*>(dn_s);
-    d.bias = dn_bias;
-    if (persist_ok(g, P) && persist_ok(d, P)) return PATH_STREAM;
-  }
-  return PATH_MX;
+  if (P > 16 * m.E && m.H % MX_BK == 0 && m.I % MX_BK == 0 && a16 && s4) return PATH_MX;
+  return PATH_AUTO;
 }
 
 static int check_shape(const MoeShape& m, const char* what) {
@@ -3632,8 +3615,7 @@ static int experts_fwd(
       (rc = check_layout(blocks_layout, down_blocks, H, I, "experts fwd (down)")))
     return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  path = resolve_path(path, m, gate_up_blocks, gate_up_scales, gate_up_bias, down_blocks, down_scales, down_bias,
-                      save_swiglu_grad != nullptr);
+  path = resolve_path(path, m, gate_up_blocks, gate_up_scales, down_blocks, down_scales, save_swiglu_grad != nullptr);
   if (noalloc) {
     workspace_bytes = carve(nullptr, T, H, I, E, k).bytes;
     BSA_REQUIRE(workspace_bytes <= NOALLOC_SCRATCH_BYTES,

@@ -203,11 +203,12 @@ class MXFP4Experts(nn.Module):
             return self._forward_in_dtype(flat, router_indices, routing_weights).reshape(shape)
         train_path = "auto"
         if self.mx_training:
-            # prefill-sized batches, widths multiples of 64, aligned blocks and scales
+            # where an inference forward would take the MX kernels: prefill-sized
+            # batches, widths multiples of 64, aligned blocks and scales
             E, I = kernels._experts_dims(self.gate_up_proj_blocks)
-            if kernels._mx_sized(flat.shape[0], router_indices.shape[-1], E, flat.shape[1], I,
-                                 self.gate_up_proj_blocks, self.gate_up_proj_scales,
-                                 self.down_proj_blocks, self.down_proj_scales):
+            if kernels._whole_forward_path("auto", flat.shape[0], router_indices.shape[-1], E, flat.shape[1], I,
+                                           self.gate_up_proj_blocks, self.gate_up_proj_scales,
+                                           self.down_proj_blocks, self.down_proj_scales) == kernels.PATHS["mx"]:
                 train_path = "mx"
         out = _MoEExperts.apply(
             flat, router_indices, routing_weights,

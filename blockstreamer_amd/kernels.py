@@ -339,32 +339,20 @@ def moe_experts_forward(hidden: Tensor, router_indices: Tensor, routing_weights:
     return out
 
 
-def _mx_sized(T: int, k: int, E: int, H: int, I: int, gu_b: Tensor, gu_s: Tensor, dn_b: Tensor, dn_s: Tensor) -> bool:
-    """Whether a batch is prefill-sized for the MX kernels (more than 16 rows
-    per expert on average) and both projections can run them: H and I
-    multiples of 64, 16-byte aligned blocks, 4-byte aligned scales."""
-    return (T * k > 16 * E and H % 64 == 0 and I % 64 == 0 and gu_b.data_ptr() % 16 == 0
-            and dn_b.data_ptr() % 16 == 0 and gu_s.data_ptr() % 4 == 0 and dn_s.data_ptr() % 4 == 0)
-
-
 def _whole_forward_path(path: str, T: int, k: int, E: int, H: int, I: int, gu_b: Tensor, gu_s: Tensor,
-                        dn_b: Tensor, dn_s: Tensor, gu_bias: Tensor | None = None,
-                        dn_bias: Tensor | None = None) -> int:
+                        dn_b: Tensor, dn_s: Tensor) -> int:
     """The path code the fused forward runs for ``path`` (the C library's
-    rule for a whole forward): "auto" takes the MX kernels for the batches of
-    ``_mx_sized``, because their gate_up stage leaves split activations for
-    their down stage, but leaves those of up to 32 rows per expert to the
-    persistent streaming kernel where both projections run it (H = I = 2880,
-    at most 256 experts, 16-byte aligned scales and biases).  (A forward saving for the
-    backward keeps the bf16 products; the stage runner never saves.)"""
+    rule for a whole forward): "auto" takes the MX kernels for prefill-sized
+    batches (more than 16 rows per expert on average) when both projections
+    can run them -- H and I multiples of 64, 16-byte aligned blocks, 4-byte
+    aligned scales -- because its gate_up stage leaves split activations for
+    its down stage.  (A forward saving for the backward keeps the bf16
+    products; the stage runner never saves.)"""
     if path != "auto":
         return PATHS[path]
-    if not _mx_sized(T, k, E, H, I, gu_b, gu_s, dn_b, dn_s):
-        return PATHS["auto"]
-    aligned = all(t is None or t.data_ptr() % 16 == 0 for t in (gu_s, dn_s, gu_bias, dn_bias))
-    if T * k <= 32 * E and H == I == 2880 and E <= 256 and T * k <= 1 << 19 and aligned:
-        return PATHS["stream"]
-    return PATHS["mx"]
+    ok = (T * k > 16 * E and H % 64 == 0 and I % 64 == 0 and gu_b.data_ptr() % 16 == 0
+          and dn_b.data_ptr() % 16 == 0 and gu_s.data_ptr() % 4 == 0 and dn_s.data_ptr() % 4 == 0)
+    return PATHS["mx"] if ok else PATHS["auto"]
 
 
 class MoEStages:
@@ -401,7 +389,7 @@ class MoEStages:
         # whole forward is resolved here, as the fused call resolves it
         self.alpha, self.limit = float(alpha), float(limit)
         self.path = _whole_forward_path(path, self.T, self.k, self.E, self.H, self.I, self.gu[0], self.gu[1],
-                                        self.dn[0], self.dn[1], gate_up_bias, down_bias)
+                                        self.dn[0], self.dn[1])
         self.ws_bytes = moe_workspace_bytes(self.T, self.H, self.I, self.E, self.k)
         self.ws = _aligned_bytes(self.ws_bytes, self.dev)
         self.out = torch.empty((self.T, self.H), dtype=torch.bfloat16, device=self.dev)

@@ -160,13 +160,10 @@ int bsa_moe_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E,
  *                   clamp masks applied (torch autograd's derivative of
  *                   gptoss.py:130-135; the reference's autograd keeps the
  *                   bf16 gate_up, the same size)
- *   path            0 = automatic (without save_swiglu_grad and where both
- *                   projections can take path 3: path 3 when more than 32 rows
- *                   per expert on average, or more than 16 unless both run the
- *                   persistent streaming kernel (H = I = 2880, at most 256
- *                   experts, 16-byte aligned scales and biases); else path 1 up
- *                   to 16 rows per expert and path 2 beyond), 1 =
- *                   weight-streaming kernel, 2 = tiled kernel,
+ *   path            0 = automatic (path 3 when more than 16 rows per expert
+ *                   on average, both projections can take it and
+ *                   save_swiglu_grad is NULL, else 1 up to 16 rows per expert and
+ *                   2 beyond), 1 = weight-streaming kernel, 2 = tiled kernel,
  *                   3 = native block-scaled MX kernel (activations split into
  *                   two MXFP8 terms by bsa_quant_mxfp8_split's rule, then two
  *                   v_mfma_scale_f32_32x32x64_f8f6f4 per 64-element k-step on

@@ -262,26 +262,22 @@ def test_combine_forms_agree_at_the_batch_limit(device, k):
     assert torch.equal(full.view(torch.int16), torch.cat(parts).view(torch.int16))
 
 
-@pytest.mark.parametrize("T,path", [(64, "auto"), (65, "stream"), (128, "stream"), (129, "mx")])
-def test_automatic_path_between_streaming_and_mx(device, T, path):
-    """8 experts, top-4, H = I = 2880: up to 16 rows per expert on average the decode rule, up to 32 the
-    persistent streaming kernel, beyond the MX kernels; a bias the streaming kernel cannot DMA moves its limit back to 16."""
+@pytest.mark.parametrize("T,path", [(64, "auto"), (65, "mx"), (128, "mx"), (129, "mx")])
+@pytest.mark.parametrize("routing", ["spread", "four experts"])
+def test_automatic_path_between_streaming_and_mx(device, T, path, routing):
+    """16 experts, top-4, H = I = 2880: up to 16 rows per expert on average the decode rule, beyond the MX kernels,
+    which read an expert's weights once per 128 rows however few experts hold the batch."""
     E, k = 16, 4
     t = synthetic.moe_layer(synthetic.MoEShape(E, k, 2880, 2880, T), seed=7, scale_lo=116, scale_hi=120, device=device)
     idx, w = synthetic.random_routing(T, E, k, seed=8, device=device)
+    if routing == "four experts":
+        idx = (torch.arange(4, device=device) * 3 + 1).expand(T, k).contiguous()
     args = expert_args(t)
-    resolved = kernels._whole_forward_path("auto", T, k, E, 2880, 2880, args[0], args[1], args[3], args[4], args[2], args[5])
+    resolved = kernels._whole_forward_path("auto", T, k, E, 2880, 2880, args[0], args[1], args[3], args[4])
     assert resolved == kernels.PATHS[path]
-    announce(f"automatic path T={T}")
+    announce(f"automatic path T={T} {routing}")
     got = kernels.moe_experts_forward(t["hidden"], idx, w, *args)
     want = kernels.moe_experts_forward(t["hidden"], idx, w, *args, path="stream" if path == "auto" else path)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     staged = kernels.MoEStages(t["hidden"], idx, w, *args).run()
     assert torch.equal(got.view(torch.int16), staged.view(torch.int16))
-    if T > 64:
-        off = torch.empty(args[2].numel() + 1, dtype=args[2].dtype, device=device)[1:].view(args[2].shape)
-        off.copy_(args[2])
-        moved = list(args)
-        moved[2] = off
-        mx = kernels.moe_experts_forward(t["hidden"], idx, w, *args, path="mx")
-        assert torch.equal(kernels.moe_experts_forward(t["hidden"], idx, w, *moved).view(torch.int16), mx.view(torch.int16))
