@@ -42,8 +42,8 @@
 //    128x128 tiles, BK=64, register-staged LDS double buffering.
 //  * moe_bwd_packed_kernel (the input-gradient backward): the packed weights
 //    read along their rows (the reduction index) and decoded in registers.
-//  * moe_bwd_stream_kernel (the same for few rows per expert): the weights
-//    from HBM to registers without LDS.  Bound: HBM.
+//  * moe_bwd_stream_kernel (the same for small batches): the weights from HBM
+//    to registers without LDS, 16 rows of an expert per workgroup.  Bound: HBM.
 // Weights are decoded with the gfx950 converter (v_cvt_scalef32_pk_bf16_fp4),
 // which follows OCP MX: a block whose E8M0 scale byte is 255 (the NaN code)
 // decodes to NaN, so the outputs it touches are NaN.  The reference's
@@ -2762,118 +2762,95 @@ __global__ __launch_bounds__(256, 1) void moe_bwd_packed_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// The same backward product for few rows per expert: the weights stream from
-// HBM straight into the registers that use them.
+// The same backward product for small batches: the weights stream from HBM
+// straight into the registers that use them.
 //
 // Bound: HBM.  The 128-row kernel above reads a weight tile through four LDS
 // stages with one wave per SIMD; with 4 rows per expert its 64 narrow LDS
 // reads and the barrier of each stage take twice the time of the stage's
-// bytes (120b layer, 128 tokens, 1.65 GB of weights: 518 us).  Here eight
-// waves own 64 rows at most and 512 columns: MG = 1, 2 or 4 groups of 16 rows
-// (the smallest that holds the rows) by MG column parts, the 8 / MG waves of
-// a part sharing out the reduction, 32 weight rows at a time in turn.  Lane
-// (c = lane & 15, g = lane >> 4) loads, for its 8 weight rows k = 8g .. 8g+7,
-// the CB = 16 / MG bytes of its own 2 CB adjacent columns and their scale
-// byte, decodes them as the 128-row kernel does and feeds
-// v_mfma_f32_16x16x32_bf16 (MFMA f's column c is the lane's column f).  No
-// weight passes through LDS and no wave waits for another until the shares
-// are added, in wave order, at the end.  320 us at 128 tokens (5.2 TB/s);
-// four waves with twice the steps in flight took 368 us (one wave per SIMD
-// leaves the decoding exposed), non-temporal loads 350 us.
+// bytes.  Here a workgroup's eight waves own 16 rows (a pass) and 512 columns
+// and share out the reduction, 32 weight rows at a time in turn.  Lane (c =
+// lane & 15, g = lane >> 4) loads, for its 8 weight rows k = 8g .. 8g+7, the
+// 16 bytes of its own 32 adjacent columns and their scale byte, decodes them
+// as the 128-row kernel does and feeds v_mfma_f32_16x16x32_bf16 (MFMA f's
+// column c is the lane's column f).  No weight passes through LDS and no wave
+// waits for another until the eight shares are added, in wave order, at the
+// end: a row's result does not depend on the rows beside it.
+//
+// Every pass of an expert is a workgroup of its own, next to each other in
+// XCD order, so that the passes of one weight tile run at the same time and
+// share its bytes in L2.  Backward of the 120b layer, 128-row kernel / this:
+// 128 tokens spread over the experts 458 / 320 us (k-pair blocks 456 / 335), on
+// 16 of them 202 / 107, on 4 230 / 91; 64 tokens spread 315 / 231.  (Passes of up
+// to 64 rows in one workgroup, with the reduction in fewer shares, took 332,
+// 225, 406 and 238 us: the long workgroups of the fuller experts are the tail.)
 // ---------------------------------------------------------------------------
-constexpr int BS_ROWS = 64;           // rows per pass
+constexpr int BS_ROWS = 16;           // rows per pass
 constexpr int BS_W = 8;               // waves
-constexpr int BS_SMEM = 128 * 1024;  // a part of every wave's float32 results
-
-template <int MG>
-struct BsCfg {
-  static constexpr int CB = 16 / MG;         // packed bytes per lane and weight row
-  static constexpr int F = 2 * CB;           // columns per lane
-  static constexpr int NCH = MG;             // column parts
-  static constexpr int KS = BS_W / NCH;      // shares of the reduction
-  static constexpr int D = MG == 1 ? 2 : 3;  // steps held in registers (256 per lane, 128 of them results)
-  static constexpr int IR = 2;               // of a lane's 4 rows, those that BS_SMEM holds at a time
-};
+constexpr int BS_D = 2;               // steps held in registers (256 per lane, 128 of them results)
+constexpr int BS_F = 32;              // columns per lane
+constexpr int BS_IR = 2;              // of a lane's 4 rows, those added at a time
+constexpr int64_t BS_MAX_TILES = 384; // workgroups of full passes up to which the kernel is taken
+constexpr int BS_SMEM = BS_W * 4 * BS_IR * BT_BN * 4;  // IR rows of every wave's float32 results
 
 // Chunk (4 columns) q's place in a row of the shares: lanes c = 0..15 writing
-// chunk j of their 4 or 8 reach 16 different places of a 256-byte LDS row.
+// chunk j of their 8 reach 16 different places of a 256-byte LDS row.
 __device__ __forceinline__ int bs_swz(int q) { return q ^ ((q >> 4) & 7); }
 
 // Raw buffers of 4-byte words (gfx9 resource word 3).  A load at BS_OOB or
 // above is out of every buffer's range: it returns 0 and reads nothing.
 constexpr int BS_RSRC = 0x00027000;
 constexpr int BS_OOB = INT32_MIN;
-template <int CB>
-__device__ __forceinline__ auto bs_load_q(__amdgpu_buffer_rsrc_t r, int v, int s) {
-  typedef uint32_t raw_t __attribute__((ext_vector_type(CB / 4)));
-  if constexpr (CB == 16)
-    return __builtin_bit_cast(raw_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
-  else if constexpr (CB == 8)
-    return __builtin_bit_cast(raw_t, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
-  else
-    return raw_t{__builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0)};
-}
 
-template <int EPI, bool KP, int MG>
+// Rows m0 .. m0 + rows - 1 (at most 16) of expert e against columns 512 nt ..
+template <int EPI, bool KP>
 __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e, int m0, int rows, int nt) {
-  using C = BsCfg<MG>;
-  constexpr int CB = C::CB, F = C::F, NCH = C::NCH, KS = C::KS, D = C::D, IR = C::IR;
-  typedef uint32_t raw_t __attribute__((ext_vector_type(CB / 4)));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15;
   const int g = lane >> 4;
-  const int ch = wave % NCH;
-  const int kw = wave / NCH;
   const int NB = a.N >> 5;
   const int64_t wrow0 = (int64_t)e * a.K;
 
   // Every address is a scalar offset of the step and row plus a lane offset
   // that never changes: buffer loads keep it in that form (one scalar add per
   // load, no vector address arithmetic).
-  const int nl = nt * BT_BN + ch * (BT_BN / NCH) + c * F;
+  const int nl = nt * BT_BN + c * BS_F;
   const int grp = min(nl >> 5, NB - 1);  // past N: the last block, not stored
-  // one expert's blocks (a whole number of 16-row bands in either layout), its scales, the tile's rows of A
+  // one expert's blocks (a whole number of 16-row bands in either layout), its scales, the pass's rows of A
   const __amdgpu_buffer_rsrc_t qb =
       __builtin_amdgcn_make_buffer_rsrc((void*)(a.Bq + wrow0 * NB * 16), 0, a.K * NB * 16, BS_RSRC);
   const __amdgpu_buffer_rsrc_t sb = __builtin_amdgcn_make_buffer_rsrc((void*)(a.Bs + wrow0 * NB), 0, a.K * NB, BS_RSRC);
   const __amdgpu_buffer_rsrc_t ab = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(a.A + (int64_t)m0 * a.lda), 0, ((rows - 1) * (int)a.lda + a.K) * 2, BS_RSRC);
   const int qrow = KP ? 32 : NB * 16;
-  const int qv = (KP ? ((g >> 1) * (NB >> 1) + (grp >> 1)) * 512 + (g & 1) * 256 + (grp & 1) * 16
-                     : (8 * g * NB + grp) * 16) +
-                 ((nl & 31) >> 1);
+  const int qv = KP ? ((g >> 1) * (NB >> 1) + (grp >> 1)) * 512 + (g & 1) * 256 + (grp & 1) * 16 : (8 * g * NB + grp) * 16;
   const int sv = 8 * g * NB + grp;
-  int av[MG];
-#pragma unroll
-  for (int m = 0; m < MG; ++m) av[m] = min(16 * m + c, rows - 1) * (int)a.lda * 2 + 16 * g;
+  const int av = min(c, rows - 1) * (int)a.lda * 2 + 16 * g;
 
   struct Step {
-    raw_t q[8];
+    u32x4_t q[8];
     uint32_t s[8];
-    s16x8_t x[MG];
+    s16x8_t x;
   };
-  const int n = ((a.K >> 5) - kw + KS - 1) / KS;  // this wave's steps
+  const int n = ((a.K >> 5) - wave + BS_W - 1) / BS_W;  // this wave's steps
   auto load = [&](Step& t, int i0) {
-    const int ks = kw + i0 * KS;
     const bool ok = i0 < n;
+    const int ks = ok ? wave + i0 * BS_W : 0;
     const int qo = ok ? qv : BS_OOB, so = ok ? sv : BS_OOB;
     const int q0 = ks * NB * 512;
     const int s0 = ks * NB * 32;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) t.q[i] = bs_load_q<CB>(qb, qo, q0 + i * qrow);
+    for (int i = 0; i < 8; ++i)
+      t.q[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(qb, qo, q0 + i * qrow, 0));
 #pragma unroll
     for (int i = 0; i < 8; ++i) t.s[i] = __builtin_amdgcn_raw_buffer_load_b8(sb, so, s0 + i * NB, 0);
-#pragma unroll
-    for (int m = 0; m < MG; ++m)
-      t.x[m] = __builtin_bit_cast(s16x8_t, __builtin_amdgcn_raw_buffer_load_b128(ab, ok ? av[m] : BS_OOB, ks * 64, 0));
+    t.x = __builtin_bit_cast(s16x8_t, __builtin_amdgcn_raw_buffer_load_b128(ab, ok ? av : BS_OOB, ks * 64, 0));
   };
-  f32x4_t acc[MG][F];
+  f32x4_t acc[BS_F];
 #pragma unroll
-  for (int m = 0; m < MG; ++m)
-#pragma unroll
-    for (int f = 0; f < F; ++f) acc[m][f] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int f = 0; f < BS_F; ++f) acc[f] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // byte B of dword w of the 8 rows -> columns 8 w + 2 B and 8 w + 2 B + 1
   auto pair = [&](const Step& t, int w, auto sel) {
     constexpr int B = decltype(sel)::value;
@@ -2885,26 +2862,23 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
       lo[d] = pack_lo16(v0, v1);
       hi[d] = pack_hi16(v0, v1);
     }
-#pragma unroll
-    for (int m = 0; m < MG; ++m) {
-      acc[m][8 * w + 2 * B] = mfma16(t.x[m], __builtin_bit_cast(s16x8_t, lo), acc[m][8 * w + 2 * B]);
-      acc[m][8 * w + 2 * B + 1] = mfma16(t.x[m], __builtin_bit_cast(s16x8_t, hi), acc[m][8 * w + 2 * B + 1]);
-    }
+    acc[8 * w + 2 * B] = mfma16(t.x, __builtin_bit_cast(s16x8_t, lo), acc[8 * w + 2 * B]);
+    acc[8 * w + 2 * B + 1] = mfma16(t.x, __builtin_bit_cast(s16x8_t, hi), acc[8 * w + 2 * B + 1]);
   };
-  Step t[D];
+  Step t[BS_D];
 #pragma unroll
-  for (int d = 0; d < D - 1; ++d) {
+  for (int d = 0; d < BS_D - 1; ++d) {
     load(t[d], d);
     __builtin_amdgcn_sched_barrier(0);  // in the loop's order, which its first wait counts on
   }
-  for (int s = 0; s < n; s += D) {
+  for (int s = 0; s < n; s += BS_D) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      load(t[(d + D - 1) % D], s + d + D - 1);
+    for (int d = 0; d < BS_D; ++d) {
+      load(t[(d + BS_D - 1) % BS_D], s + d + BS_D - 1);
       // no step's decoding moves up between another's loads
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int w = 0; w < CB / 4; ++w) {
+      for (int w = 0; w < 4; ++w) {
         pair(t[d], w, std::integral_constant<int, 0>{});
         pair(t[d], w, std::integral_constant<int, 1>{});
         pair(t[d], w, std::integral_constant<int, 2>{});
@@ -2916,14 +2890,14 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
 
   int te = tid;  // the epilogue's addresses are not worth registers during the loop
   asm volatile("" : "+v"(te));
-  // The shares are added IR of every lane's four rows at a time: [share][4 MG
-  // IR rows][128 chunks], then each thread sums and stores 4 columns of a row.
-  constexpr int NR = 4 * MG * IR;
+  // The shares are added IR of every lane's four rows at a time: [share][4 IR
+  // rows][128 chunks], then each thread sums and stores 4 columns of a row.
+  constexpr int IR = BS_IR;
+  constexpr int NR = 4 * IR;
   constexpr int IT = NR * 2 / BS_W;  // 4-column pieces per thread
-  static_assert(KS * NR * BT_BN * 4 <= BS_SMEM, "shares");
 #pragma unroll
   for (int h = 0; h < 4; h += IR) {
-    // local row lr of this part -> row of the tile
+    // local row lr of this part -> row of the pass
     auto row_of = [&](int lr) { return 4 * (lr / IR) + h + lr % IR; };
     u32x4_t fac[IT];
     if constexpr (EPI == EPI_SWIGLU_BWD) {
@@ -2936,17 +2910,15 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
     }
     __syncthreads();
 #pragma unroll
-    for (int m = 0; m < MG; ++m)
+    for (int i = 0; i < IR; ++i)
 #pragma unroll
-      for (int i = 0; i < IR; ++i)
-#pragma unroll
-        for (int j = 0; j < F / 4; ++j) {
-          const int q = (ch * (BT_BN / NCH) + (te & 15) * F) / 4 + j;
-          const int lr = (4 * m + ((te >> 4) & 3)) * IR + i;
-          const int v = h + i;
-          *reinterpret_cast<f32x4_t*>(smem + ((kw * NR + lr) * 128 + bs_swz(q)) * 16) =
-              f32x4_t{acc[m][4 * j][v], acc[m][4 * j + 1][v], acc[m][4 * j + 2][v], acc[m][4 * j + 3][v]};
-        }
+      for (int j = 0; j < BS_F / 4; ++j) {
+        const int q = (te & 15) * BS_F / 4 + j;
+        const int lr = ((te >> 4) & 3) * IR + i;
+        const int v = h + i;
+        *reinterpret_cast<f32x4_t*>(smem + ((wave * NR + lr) * 128 + bs_swz(q)) * 16) =
+            f32x4_t{acc[4 * j][v], acc[4 * j + 1][v], acc[4 * j + 2][v], acc[4 * j + 3][v]};
+      }
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
@@ -2957,7 +2929,7 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
       if (r >= rows || col >= a.N) continue;
       f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < KS; ++k) o += *reinterpret_cast<const f32x4_t*>(smem + ((k * NR + lr) * 128 + bs_swz(q)) * 16);
+      for (int k = 0; k < BS_W; ++k) o += *reinterpret_cast<const f32x4_t*>(smem + ((k * NR + lr) * 128 + bs_swz(q)) * 16);
       const float v[4] = {o[0], o[1], o[2], o[3]};
       bt_store4<EPI>(a, m0 + r, col, v, fac[it]);
     }
@@ -2967,21 +2939,39 @@ __device__ __forceinline__ void bs_tile(const GemmArgs& a, uint8_t* smem, int e,
 template <int EPI, bool KP>
 __global__ __launch_bounds__(64 * BS_W) void moe_bwd_stream_kernel(GemmArgs a) {
   extern __shared__ __align__(1024) uint8_t smem[];  // BS_SMEM
-  const int L = xcd_tile_index(*a.num_tiles * a.n_tiles_n);
+  const int lane = threadIdx.x & 63;
+  // The tiles (pass, column tile) in expert order, an expert's column tiles
+  // one after the other, each for all of its passes.  Every wave finds its
+  // workgroup's by itself, lane l looking at experts l, l + 64, ...
+  auto passes = [&](int ex) { return ex < a.E ? (a.counts[ex] + BS_ROWS - 1) / BS_ROWS : 0; };
+  int live = 0;
+  for (int e0 = 0; e0 < a.E; e0 += 64) live += passes(e0 + lane);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) live += __shfl_xor(live, off);
+  const int L = xcd_tile_index(__builtin_amdgcn_readfirstlane(live) * a.n_tiles_n);
   if (L < 0) return;
-  int tile, nt;
-  tile_of<TL_BM>(a, L, tile, nt);
-  const int2 te = a.tiles[tile];
-  const int e = te.x;
-  const int end = min(te.y + TL_BM, a.offsets[e] + a.counts[e]);
-  for (int m0 = te.y; m0 < end; m0 += BS_ROWS) {
-    const int rows = min(BS_ROWS, end - m0);
-    if (rows <= 16)
-      bs_tile<EPI, KP, 1>(a, smem, e, m0, rows, nt);
-    else if (rows <= 32)
-      bs_tile<EPI, KP, 2>(a, smem, e, m0, rows, nt);
-    else
-      bs_tile<EPI, KP, 4>(a, smem, e, m0, rows, nt);
+  const int q = L / a.n_tiles_n;
+  int before = 0;  // passes of the experts before the 64 looked at
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int np = passes(e0 + lane);
+    int incl = np;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off);
+      if (lane >= off) incl += v;
+    }
+    const uint64_t past = __ballot(before + incl > q);
+    if (past) {
+      const int i = __builtin_ctzll(past);
+      const int e = e0 + i;
+      const int c = __builtin_amdgcn_readlane(np, i);
+      const int r = L - (before + __builtin_amdgcn_readlane(incl, i) - c) * a.n_tiles_n;
+      const int nt = r / c;
+      const int m = BS_ROWS * (r - nt * c);
+      bs_tile<EPI, KP>(a, smem, e, a.offsets[e] + m, min(BS_ROWS, a.counts[e] - m), nt);
+      return;
+    }
+    before += __builtin_amdgcn_readlane(incl, 63);
   }
 }
 
@@ -3028,18 +3018,23 @@ static int launch_gemm_packed_rows(const GemmArgs& a, int64_t P, hipStream_t st)
     return BSA_EINVAL;
   }
   // Few rows per expert: the streaming kernel, whose 32-bit offsets need an
-  // expert's blocks and 64 rows of A below 2 GiB.  Forward + backward of the
-  // 120b layer, this kernel against the 128-row one: 8 rows per expert (256
-  // tokens) 787 / 866 us, 16 (512) 1069 / 1157, 24 (760) 1624 / 1276; with 32
-  // experts, whose tiles leave a quarter of the CUs idle, 8 (64) 250 / 273, 16
-  // (128) 382 / 345.  One expert (mxfp4_matmul's transposed product, 5760 x
-  // 2880): 1 to 8 rows 44 / 100 us.
+  // expert's blocks and 16 rows of A below 2 GiB.  The host knows the rows of
+  // an expert on average only, and what the kernel costs is its passes: P / 16
+  // where few experts hold the batch, at most one more per expert.  So the line
+  // is drawn at the workgroups that full passes make (384: 1024 rows at 2880
+  // columns); beyond it batches on some tens of experts lose (backward of the 120b
+  // layer, 128-row kernel / this, spread over all experts, on 64, on 32, on 16
+  // of them: 256 tokens 487 / 401, 320 / 297, 209 / 191, 231 / 165 us; 320
+  // tokens 508 / 407, 333 / 295, 215 / 255, 241 / 200; 32 experts: 128 tokens
+  // 205 / 193, on 8 of them 228 / 92).  One expert (mxfp4_matmul's transposed
+  // product, 5760 x 2880): 1 to 16 rows 99 / 42.
   const bool b32 = (int64_t)a.K * a.N / 2 <= INT32_MAX && (int64_t)BS_ROWS * a.lda * 2 <= INT32_MAX;
-  if (q16 && b32 && P <= (a.E == 1 || (int64_t)a.E * b.n_tiles_n >= 512 ? 16 : 8) * (int64_t)a.E) {
+  if (q16 && b32 && P <= 16 * (int64_t)a.E && P * b.n_tiles_n <= BS_MAX_TILES * BS_ROWS) {
     void (*fn)(GemmArgs) = a.kp ? moe_bwd_stream_kernel<EPI, true> : moe_bwd_stream_kernel<EPI, false>;
     int rc = allow_big_lds(reinterpret_cast<const void*>(fn), a.kp ? 10 : 9, EPI, BS_SMEM);
     if (rc) return rc;
-    hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(64 * BS_W), BS_SMEM, st, b);
+    const int64_t passes = std::min<int64_t>(P, P / BS_ROWS + a.E);
+    hipLaunchKernelGGL(fn, dim3((unsigned)align_up(passes * b.n_tiles_n, 8)), dim3(64 * BS_W), BS_SMEM, st, b);
     BSA_LAUNCH_CHECK("streaming backward GEMM launch");
     return BSA_OK;
   }

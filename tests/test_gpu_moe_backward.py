@@ -55,6 +55,8 @@ CASES = [
     (16, 4, 512, 256, 129, 116, 120),
     (4, 1, 128, 192, 77, 117, 121),
     (4, 2, 64, 32, 5, 117, 121),   # one k-tile in both products, one column block
+    (4, 2, 64, 32, 40, 117, 121),  # the same with more than 16 rows per expert: the 128-row kernel
+    (8, 2, 256, 256, 65, 116, 120),
 ]
 
 
@@ -75,10 +77,12 @@ def test_backward_vs_oracle_autograd(device, case):
 
 
 @pytest.mark.parametrize("layout", ["checkpoint", "kpair"])
-@pytest.mark.parametrize("H,I", [(640, 576), (576, 544), (64, 32)], ids=["H640I576", "H576I544", "H64I32"])
+@pytest.mark.parametrize("H,I", [(640, 576), (576, 544), (64, 32), (128, 1088), (1088, 64)],
+                         ids=["H640I576", "H576I544", "H64I32", "H128I1088", "H1088I64"])
 def test_backward_few_rows_per_expert(device, H, I, layout):
-    """The streaming backward kernel at the edges of its 16-row groups and 64-row passes, beside experts
-    without rows, with column tiles of 512 columns and a rest, and with fewer k-steps than waves."""
+    """The streaming backward kernel at the edges of its 16-row passes, beside experts without rows,
+    with column tiles of 512 columns and a rest, and with fewer k-steps than waves.  A token's
+    gradient does not depend on the rows beside it: alone it has the same bits."""
     if layout == "kpair" and I % 64:
         pytest.skip("the k-pair layout needs an even number of 32-element groups")
     counts = [1, 16, 17, 0, 32, 33, 64, 65]
@@ -92,6 +96,32 @@ def test_backward_few_rows_per_expert(device, H, I, layout):
     g = torch.randn(T, H, generator=gen).to(torch.bfloat16).to(device)
     announce(f"moe backward, few rows per expert, {H} x {I}, {layout}")
     _, rh, rw = _oracle_grads(t, idx, w, g)
+    if layout == "kpair":
+        for name in ("gate_up_proj_blocks", "down_proj_blocks"):
+            t[name] = kernels.to_kpair(t[name])
+    _, gh, gw = _gpu_grads(t, idx, w, g)
+    assert_grad_close(gh, rh, "d hidden")
+    assert_grad_close(gw, rw, "d routing weights")
+    for i in range(0, T, 29):
+        one = dict(t, hidden=t["hidden"][i:i + 1])
+        _, oh, ow = _gpu_grads(one, idx[i:i + 1], w[i:i + 1], g[i:i + 1])
+        assert torch.equal(oh.view(torch.int16), gh[i:i + 1].view(torch.int16)), i
+        assert torch.equal(ow, gw[i:i + 1]), i
+
+
+@pytest.mark.parametrize("layout", ["checkpoint", "kpair"])
+@pytest.mark.parametrize("E,T,held", [(128, 64, 128), (128, 255, 128), (128, 256, 32), (128, 257, 16), (32, 127, 32),
+                                      (32, 128, 4), (32, 129, 8)])
+def test_backward_2880_either_side_of_the_streaming_line(device, E, T, held, layout):
+    """The gpt-oss widths on both sides of the lines of the streaming backward kernel (1024 rows, 16 per expert), the
+    batch spread over the experts or held by some of them, against float32 autograd."""
+    k = 4
+    t = synthetic.moe_layer(synthetic.MoEShape(E, k, 2880, 2880, T), seed=E + T, scale_lo=116, scale_hi=120, device=device)
+    idx, w = synthetic.random_routing(T, held, k, seed=T, dtype=torch.float32, device=device)
+    idx = (idx + 1) * (E // held) - 1
+    g = (torch.randn(T, 2880, generator=torch.Generator().manual_seed(T)) * 0.1).to(torch.bfloat16).to(device)
+    announce(f"moe backward 2880, E={E} T={T} on {held} experts, {layout}")
+    rh, rw = _gpu_fp32_reference_grads(t, idx, w, g)
     if layout == "kpair":
         for name in ("gate_up_proj_blocks", "down_proj_blocks"):
             t[name] = kernels.to_kpair(t[name])
@@ -235,13 +265,13 @@ def test_mxfp4_matmul_gradient_and_memory(device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("rows", [5, 200])
+@pytest.mark.parametrize("rows", [5, 9, 16, 17, 200])
 def test_mxfp4_matmul_gptoss_shape(device, dtype, rows):
     """gpt-oss gate_up weight (N = 5760 rows of K = 2880): the forward and the
     input gradient against float64 products of the exact weight, to the
     output dtype's rounding plus the float32 summation bound; the k-pair
-    layout gives the same bits.  5 rows run the weight-streaming kernels, 200
-    the tiled ones."""
+    layout gives the same bits.  Up to 16 rows run the weight-streaming kernels,
+    17 and more the tiled ones."""
     b, s = synthetic.packed_weights(1, 5760, 90, seed=rows, scale_lo=116, scale_hi=121, device=device)
     w = gptoss.dequantize_expert(b, s, torch.float32).double()
     g = torch.Generator().manual_seed(rows + 1)
