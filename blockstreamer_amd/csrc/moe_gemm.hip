@@ -811,9 +811,9 @@ __global__ __launch_bounds__(256, 3) void moe_stream_parts_kernel(GemmArgs a) {
 
 // ---------------------------------------------------------------------------
 // Persistent weight-streaming kernel (decode and short prompts) for a K =
-// 32*G known at compile time.  Persistent workgroups, two per CU, each walk a
-// contiguous run of work items; an item is 16 weight rows (one 16-column MFMA
-// block) of one expert against one pass of that expert's sorted rows, items
+// 32*G known at compile time.  Persistent workgroups, two per CU (one where
+// RG is 2), each walk a contiguous run of work items; an item is 16 weight rows
+// (one 16-column MFMA block) of one expert against one pass of that expert's sorted rows, items
 // ordered by (hit expert, pass, weight-row slice).  Consecutive items of a
 // workgroup share the expert, so the A operands stay in registers and are
 // reloaded only when the (expert, pass) changes.
@@ -3143,14 +3143,17 @@ static int run_dispatch(const int64_t* idx, int64_t P, int E, const Workspace& w
 }
 
 // Row groups (16-row blocks sharing one read of the weights) of the
-// persistent kernel: two once experts commonly hold more than 16 rows.  120b
-// layer, one against two (unevenly hit experts): 64 tokens 199 / 218 us, 128
-// 245 / 252, 256 338 / 325, 512 514 / 420; on k-pair blocks 200 tokens 297 /
-// 310.  With few experts the line lies later: 32 experts, 66 tokens 105 / 120
-// us, 72 116 / 120, 80 121 / 119, 128 144 / 132.  (Four waves' operands of 32
-// rows do not fit a wave's registers, so two groups take 512 threads and the CU's
-// whole ring, which the smaller batches, with fewer rows to share, pay for.)
-static int ps_row_groups(int64_t P, int64_t E) { return P > (E >= 64 ? 8 : 10) * E ? 2 : 1; }
+// persistent kernel: two once experts commonly hold more than 16 rows and
+// there are passes enough to share.  One against two, 120b layer: 192 tokens
+// 294 / 302 us, 256 333 / 324, 320 380 / 349, 512 496 / 424; 64 experts: 128 tokens
+// 178 / 184, 160 198 / 194; 32 experts: 80 tokens 110 / 117 (on 4 of them 69 /
+// 76), 112 125 / 129 (82 / 87), 120 131 / 133 (100 / 88); 16 experts: 64 tokens
+// 77 / 84.  (Four waves' operands of 32 rows do not fit a wave's registers, so
+// two groups take 512 threads and the CU's whole ring, which the smaller
+// batches, with fewer rows to share, pay for.)  A single expert's product
+// (mxfp4_matmul, 5760 x 2880) has fewer items than workgroups either way: 12
+// rows 17.5 / 15.2 us.
+static int ps_row_groups(int64_t P, int64_t E) { return P > (E == 1 ? 10 : std::max<int64_t>(8 * E, 448)) ? 2 : 1; }
 
 template <int EPI, int RG>
 static int launch_persist(const GemmArgs& a, int cus, hipStream_t st) {

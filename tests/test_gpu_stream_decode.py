@@ -144,14 +144,14 @@ def test_persistent_two_row_groups_edges(device, rows):
     a group and of a pass, against the part kernel and the oracle.  A token's row does
     not depend on the batch: the same tokens one by one (one row group) give the same bits."""
     E, k = 8, 1
-    counts = [rows[0], rows[1], 0, 32, 16, 1, 48, 31]
+    counts = [rows[0], rows[1], 0, 32, 16, 1, 449, 31]
     T = sum(counts)
     t = synthetic.moe_layer(synthetic.MoEShape(E, k, 2880, 2880, T), seed=61, scale_lo=116, scale_hi=120,
                             device=device)
     idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(
         T, generator=torch.Generator().manual_seed(1))].reshape(T, k).to(device)
     w = torch.full((T, k), 0.5, dtype=torch.bfloat16, device=device)
-    assert T * k > 8 * E
+    assert T * k > max(8 * E, 448)  # two row groups; the tokens taken one by one below run one
     announce(f"persistent kernel, two row groups, counts {counts}")
     persist, parts = _both_kernels(t, idx, w)
     _agree(persist, parts, f"counts {counts}")
@@ -162,3 +162,15 @@ def test_persistent_two_row_groups_edges(device, rows):
         one = kernels.moe_experts_forward(t["hidden"][i:i + 1], idx[i:i + 1], w[i:i + 1], *expert_args(t),
                                           path="stream")
         assert torch.equal(one.view(torch.int16), persist[i:i + 1].view(torch.int16))
+
+
+@pytest.mark.parametrize("E,k,T", [(16, 4, 113), (32, 4, 113), (64, 4, 129)])
+def test_persistent_row_group_line(device, E, k, T):
+    """One token more than the last batch with one row group per workgroup: every other token keeps its bits."""
+    t = synthetic.moe_layer(synthetic.MoEShape(E, k, 2880, 2880, T), seed=E, scale_lo=116, scale_hi=120, device=device)
+    idx, w = synthetic.random_routing(T, E, k, seed=T, device=device)
+    assert T * k > max(8 * E, 448) >= (T - 1) * k
+    announce(f"persistent kernel, row group line, E={E}")
+    two = kernels.moe_experts_forward(t["hidden"], idx, w, *expert_args(t), path="stream")
+    one = kernels.moe_experts_forward(t["hidden"][:-1], idx[:-1], w[:-1], *expert_args(t), path="stream")
+    assert torch.equal(one.view(torch.int16), two[:-1].view(torch.int16))
