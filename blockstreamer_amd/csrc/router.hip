@@ -435,11 +435,14 @@ extern "C" int bsa_router_fwd(const void* hidden, int dtype, int64_t T, int64_t 
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (mfma) {
     // logits tiles, then top-k + softmax from the (L2-resident) logits
-    if (T >= 4096 && (T > 4096 || E <= 64) && E <= RF_MAX_E && H <= (1 << 20)) {
+    if (T >= 4096 && (T > 4096 || E <= 64) && E <= RF_MAX_E && H <= 4096) {
       // The whole router in one launch.  Norm + router against the separate
       // launches: 128 experts, 8192 tokens 60 / 65 us, 5000 54 / 59, but 4096
       // 54 / 47: there their 256 workgroups are one per CU.  32 experts: 8192
-      // tokens 42 / 50, 4096 38 / 44.
+      // tokens 42 / 50, 4096 38 / 44; the router alone, 4097 tokens, 64 experts
+      // 26 / 28, 48 24 / 25, 33 22 / 26.  Every workgroup reads the whole weight, so
+      // wide rows take the launches: 4097 tokens, 4096 wide, 128 experts 50 / 50,
+      // 7168 wide 81 / 76, 64 experts 56 / 53.
       const dim3 grid((unsigned)((T + 31) / 32));
       auto fn = E <= 32 ? router_fused_kernel<1> : (E <= 64 ? router_fused_kernel<2> : router_fused_kernel<4>);
       hipLaunchKernelGGL(fn, grid, dim3(512), 0, st, static_cast<const uint16_t*>(hidden),

@@ -91,7 +91,7 @@ def test_router_bf16_module(device, T, E, k):
 
 
 @pytest.mark.parametrize("T,H,E,k", [(4128, 2880, 128, 4), (4097, 160, 32, 4), (4111, 32, 5, 5), (4130, 96, 33, 3),
-                                     (4096, 288, 64, 8), (4099, 640, 100, 16)])
+                                     (4096, 288, 64, 8), (4099, 640, 100, 16), (4097, 4096, 48, 4), (4097, 4128, 48, 4)])
 def test_router_one_launch(device, T, H, E, k):
     """The one-launch router of long prompts: token and expert remainders, fewer k-steps than a wave's
     loads in flight, ties, infinities and NaN.  More than 128 experts take the separate kernels, whose
