@@ -166,7 +166,9 @@ __device__ __forceinline__ void wait_vmcnt_tiles(int ahead) {
 // read, i.e. for the next tile in the middle of the present one.  It counts no
 // destination registers, so the kernels' own vmcnt waits and barriers are all
 // that orders it; a vmcnt wait the compiler adds for loads of its own can
-// only wait for more than it needs.
+// only wait for more than it needs.  m0 is a reserved register that no clobber
+// list can name: nothing else in these kernels may need it (an LDS DMA builtin
+// beside them would, and the compiler could keep its m0 across this one).
 __device__ __forceinline__ void at_dma16(const void* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
 }
@@ -818,7 +820,7 @@ __device__ __forceinline__ void at_dkv_unit(const uint8_t* T, bool full, uint32_
 // see one of its keys (R = t * G + i as in the forward) in units of 32,
 // through a DMA ring: the q and dO tiles (rows permuted as A operands;
 // q^T and dO^T by transposing reads for dv^T += dO^T P and dk^T += q^T dS) and
-// the rows' (L, D).  Four waves with no common rows keep no sums to add at the
+// the rows' (L, D).  Four waves with no common keys keep no sums to add at the
 // end, and at 167 registers three workgroups share a CU, out of step with each
 // other: one's MFMAs run under another's exponentials, where the eight waves
 // of one workgroup met at the same barrier.  4096 causal tokens, 64/8 heads:

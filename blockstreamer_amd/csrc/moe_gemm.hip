@@ -18,10 +18,10 @@
 //
 // Kernels:
 //  * moe_stream_persist_kernel (decode, K = 2880): persistent workgroups,
-//    two per CU, walking (expert, 16-row pass, 16-weight-row slice) items
+//    walking (expert, pass of 16 or 32 rows, 16-weight-row slice) items
 //    through LDS DMA rings; the packed weights go to the block-scaled MFMA
 //    as they are, against the activations split into two MXFP8 terms.
-//    Bound: HBM (each hit expert's weights are read exactly once).
+//    Bound: HBM (a hit expert's weights are read once per pass).
 //  * moe_stream_parts_kernel (decode, K = 2880 with operands the persistent
 //    kernel cannot DMA) and moe_stream_kernel (decode, any other K): one
 //    workgroup per (expert, column slice), weights decoded to bf16 for
@@ -35,9 +35,9 @@
 //    expert on average):
 //    128x256 tiles of one expert on the block-scaled
 //    v_mfma_scale_f32_32x32x64_f8f6f4, the packed weights as they are
-//    against activations split into two MXFP8 terms (hi, lo), two stages
-//    of global_load_lds DMA and LDS reads issued half a step ahead of the
-//    MFMAs (mx_split_step).  Bound: MFMA issue and the L2->LDS stream.
+//    against activations split into two MXFP8 terms (hi, lo), DMA stages of
+//    one step (activations) and two (weights), LDS reads issued half a step
+//    ahead of the MFMAs (mx_split_step).  Bound: MFMA issue and the L2->LDS stream.
 //  * moe_tiled_kernel (prefill for operands aligned to less than 16 bytes):
 //    128x128 tiles, BK=64, register-staged LDS double buffering.
 //  * moe_bwd_packed_kernel (the input-gradient backward): the packed weights
@@ -1754,26 +1754,25 @@ __global__ __launch_bounds__(256, 2) void moe_tiled2_kernel(GemmArgs a) {
 // 16g .. 16g+15 (bytes 0-15) and 32+16g .. 32+16g+15 (bytes 16-31), while
 // its scale byte is still the scale of K block g.
 //
-// Tile 128 rows x BN weight rows, BK = 64 (two MX blocks), NS LDS stages
-// filled only by global_load_lds DMA, every DMA covering whole contiguous
-// runs:
+// Tile 128 rows x 256 weight rows, BK = 64 (two MX blocks), LDS stages (laid
+// out below) filled only by global_load_lds DMA, every DMA covering whole
+// contiguous runs:
 //  * A stage [128][128 B]: per row the k-tile's 64 hi codes then 64 lo codes
 //    (the split's row layout), 8 lanes per row; row r's 16-byte chunk c sits
 //    at chunk c ^ ((r >> 1) & 7), so the fragment reads are bank-conflict
 //    free (ds_read_b128 serves 16 lanes a cycle from 64 banks, i.e. 256
 //    bytes: two 128-byte rows share the banks, so the swizzle pairs them);
-//  * B stage [BN rows][2 groups][16 bytes], 2 lanes per row (32 contiguous
-//    bytes, 512 in the k-pair layout), the two halves of row q swapped when
-//    bit 3 of q is set;
+//  * B stage of two k-steps, 4 lanes per row (64 contiguous bytes; 1 KiB per
+//    16 rows in the k-pair layout);
 //  * A scales, 4 B per row, per stage: the split writes the activations
 //    k-tile-major (k-tile kt of sorted row p at kt*ldq + 128p, its two scale
 //    bytes at kt*ldas + 4p), so a stage's codes and scales are each one
 //    contiguous run; lo's scale byte is hi's minus 4;
-//  * the B scales of the tile's BN weight rows, one contiguous BN*G-byte
-//    span of the checkpoint tensor, are loaded once per tile.
-// A 2 x WN grid of waves (default 2 x 2: each wave 64 rows x 128 weight rows,
-// 2 x 4 blocks of 32 x 32, two workgroups per CU) splits the tile; 64 x 128
-// per wave reads 12 LDS fragments per 16 MFMAs where 128 x 64 reads 18.
+//  * B scales in chunks of 12 steps.
+// A 2 x 2 grid of waves (each wave 64 rows x 128 weight rows, 2 x 4 blocks of
+// 32 x 32, two workgroups per CU) splits the tile; 64 x 128 per wave reads 12
+// LDS fragments per 16 MFMAs where 128 x 64 reads 18.  Tiles of at most 64 rows
+// take a form of their own (thin tiles, below).
 // Bound: the L2-to-LDS DMA rate and MFMA issue at the FP8 rate (two
 // instructions per step: the bf16 rate), each alone close to the whole.
 // ---------------------------------------------------------------------------
@@ -3051,7 +3050,7 @@ static int launch_gemm_packed_rows(const GemmArgs& a, int64_t P, hipStream_t st)
 constexpr int T2_LAUNCH_NS = 2;  // and of the launched bf16 tiled kernel
 
 // Kernels using more than 64 KiB of dynamic LDS must be allowed to, once per
-// kernel and device.  `kind` (0..7) x `epi` (0..3) names the kernel.
+// kernel and device.  `kind` (0..15) x `epi` (0..7) names the kernel.
 static int allow_big_lds(const void* fn, int kind, int epi, int bytes = 160 * 1024) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {

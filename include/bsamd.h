@@ -432,7 +432,9 @@ int bsa_rmsnorm_bwd(const void *grad_out, const void *x, int dtype, int64_t T,
  * sinks: float32 [Hq], or null for no sink.  Masks: causal = 0 shows every
  * key (what the eager path does with attention_mask = None); causal = 1 shows
  * key j to query t when j <= Tk - Tq + t, and window > 0 also requires
- * Tk - Tq + t - j < window.  lse (optional, float32 [B, Hq, Tq]) receives
+ * Tk - Tq + t - j < window (a window of Tk or more is none).  scaling must be
+ * positive where a mask hides a key or Tk is no multiple of 64.  lse (optional,
+ * float32 [B, Hq, Tq]) receives
  * log2 of each row's softmax denominator (sink included) in units of
  * scaling * log2(e) times the dot products: what bsa_attention_bwd needs.
  * Float32 accumulation; probabilities rounded to bf16 for the value product.
